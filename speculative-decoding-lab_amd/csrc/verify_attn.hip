@@ -266,6 +266,21 @@ __host__ __device__ constexpr int ring_depth(int, int, int) { return 2; }
 // and spill fixes), scaled to the page size.
 __host__ __device__ constexpr int piece_cost(int d, int kt) { return 32 * 8192 / (16 * d * 2 * (kt == SPV_FP8E4M3 ? 1 : 2)); }
 constexpr int kMfmaThreads = 512;
+// The smallest piece of the equal-pieces split, in pages, for a longest
+// context of `maxnp` pages: cutting finer than fills the workgroups' waves
+// only adds partials. A piece of 16 pages gives each of the eight waves two; a
+// segment of np pages in pieces of P costs about t_page P / 8 of walk and
+// t_merge np / (8 P) of the last arriver's merge (kMergeChunk slots a round
+// trip), least near P = sqrt(np t_merge / t_page) -- 2 sqrt(np) measured.
+// Without the bound a small batch was cut into pieces of one or two pages and
+// merges of up to 256 slots (planned calls, us, without / with): batch 8 of 64
+// to 1,024 keys, 12/2 heads of 128, 30.8 / 14.5; one sequence of 4,096 keys
+// 40.1 / 15.8, of 16,384 66.6 / 28.5; two of 32,768 over fp8 pages, 14/2
+// heads of 64, 45.9 / 30.4; one-row decode of 1,000 keys 20.5 / 6.4. (Floors
+// of 8 and 32 pages: 14.3 and 14.4 at the first shape, 7.4 and 7.8 at the
+// last; 1.4 sqrt and 2.8 sqrt: 28.0 and 29.8 at 16,384 keys.) Batches that
+// fill the grid with longer pieces than this are cut as before.
+__device__ __forceinline__ int min_piece(int maxnp) { return max(16, (int)(2.f * __builtin_sqrtf((float)maxnp))); }
 // O^T tiles combined per LDS round: as many as fit beside the other buffers
 // (the slots take 8 waves x 16 * nt rows x 64 B per tile). With four query
 // tiles: all four of head_dim 64 in one round (long context 2 us faster than
@@ -373,7 +388,8 @@ __device__ __forceinline__ int ceil_div(int a, int P, float rP) {
 // is cut into k = ceil(np / P) near-equal page ranges, with P chosen so that
 // HR * sum_b k_b <= nw: each workgroup then holds at most one piece and pays
 // the per-piece costs (query staging, wave combine, partial, merge) once.
-// P starts at ceil(total / nw) and grows in proportion to the overshoot;
+// P starts at ceil(total / nw), at least min_piece, and grows in proportion
+// to the overshoot;
 // when the segments alone outnumber the workgroups, P is the longest context
 // and every piece is a whole segment. Wave 0 computes the whole plan with
 // wave-wide scans (no barrier until the end), and keeps each sequence's id
@@ -414,7 +430,8 @@ __device__ void build_plan(const AttnParams& p, int* s_pref, int* s_kpref, int* 
     if constexpr (!BAL) {
     auto pages_of = [&](int b) { return one ? np1 : s_pref[b + 1] - s_pref[b]; };
     const long long T = HR * carry;
-    int P = HR * p.B >= nw ? maxnp : (int)min((long long)maxnp, max(1LL, div_floor(T + nw - 1, nw)));
+    int P = HR * p.B >= nw ? maxnp
+                           : (int)min((long long)maxnp, max((long long)min_piece(maxnp), div_floor(T + nw - 1, nw)));
     int npieces;
     for (;;) {
       const float rP = __builtin_amdgcn_rcpf((float)P);

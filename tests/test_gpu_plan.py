@@ -136,3 +136,22 @@ def test_plan_reports_unwritten_keys(cuda):
     assert gpu.seq_lengths == [306, 506]
     with pytest.raises(ValueError, match="does not match its plan"):
         verify_attention(q, gpu, 0, [0, 1], lens, 700, plan=plan)
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,d,C,lo,hi", [
+    (1, 12, 2, 128, 6, 250, 250),      # one page less than, or exactly, one smallest piece (16 pages)
+    (1, 12, 2, 128, 6, 251, 251),      # one page more: two pieces
+    (2, 14, 2, 64, 1, 1017, 1030),     # the floor meets 2 sqrt(pages) at 64 pages, one row
+    (1, 12, 2, 128, 4, 16000, 16000),  # pieces of 63 pages: 16 partials, two merge round trips
+    (3, 16, 2, 128, 9, 3, 9000),       # four query tiles and two row groups, one context far longer
+])
+def test_smallest_piece_of_the_equal_split(cuda, B, Hq, Hkv, d, C, lo, hi):
+    lens = [hi] + _lens(B - 1, lo, hi, seed=B + hi)
+    gpu, keys, values = _dense_pool(cuda, lens, C, Hkv, d, 16, torch.bfloat16, seed=B + C)
+    q = torch.randn(B, C, Hq, d, generator=torch.Generator().manual_seed(hi)).to(torch.bfloat16)
+    qd, sids, max_ctx = q.to(cuda), list(range(B)), max(lens) + C
+    plain = verify_attention(qd, gpu, 0, sids, lens, max_ctx)
+    plan = VerifyPlan(gpu, sids, lens, C, Hq, max_ctx)
+    for _ in range(2):  # the arrival counters are left at zero
+        assert torch.equal(verify_attention(qd, gpu, 0, sids, lens, max_ctx, plan=plan), plain)
+    _bf16_check(plain, ref_attn.extend_attention_dense(q.float(), keys, values, lens, Hq))
