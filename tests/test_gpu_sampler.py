@@ -419,3 +419,32 @@ def test_workspace_reused_across_batch_sizes(cuda):
         want = S.verify_from_logits(target, draft, x, u, noise, 1.0)
         res = es.verify_sample(target.to(cuda), draft.to(cuda), x.to(cuda), u.to(cuda), noise.to(cuda), 1.0)
         assert res.accepted_lists() == want, B
+
+
+@pytest.mark.parametrize("V", [50257, 151936])
+@pytest.mark.parametrize("a,b", [(0, 10239), (10239, 10240), (20480, -1), (-2, -1)])
+@pytest.mark.parametrize("reject", [True, False])
+def test_exact_race_visits_every_contending_chunk(cuda, V, a, b, reject):
+    """Two equal best keys at the edges of the race's chunks (10,240 entries,
+    the last one short), and a third just below in another chunk: the exact
+    re-race must see both, keep the lower index and flag the draw; with the
+    second key one part in 10^3 larger it wins unflagged."""
+    a, b = a % V, b % V
+    gamma = 1
+    g = torch.Generator().manual_seed(V + a)
+    p = torch.rand(1, gamma + 1, V, generator=g)
+    q = torch.rand(1, gamma, V, generator=g)
+    row = 0 if reject else gamma
+    p[0, row, a] = p[0, row, b] = 0.5
+    q[0, 0, a] = q[0, 0, b] = 0.0
+    noise = torch.empty(1, V).exponential_(1, generator=g).clamp_min_(1e-3)
+    noise[0, a] = noise[0, b] = 2.0 ** -30
+    x = torch.tensor([[7]], dtype=torch.int32)
+    u = torch.full((1, 1), 2.0 if reject else 0.0)
+    for scale, token, flag in ((1.0, a, _hip.FLAG_DRAW_BAND), (0.999, b, 0)):
+        e = noise.clone()
+        e[0, b] *= scale
+        res = es.verify_sample(p.to(cuda), q.to(cuda), x.to(cuda), u.to(cuda), e.to(cuda), 1.0, is_probs=True)
+        assert res.accepted_lists() == [[token] if reject else [7, token]]
+        assert res.accepted_lists() == S.batch_accept_noise(p, q, x, u, e)
+        assert res.flags.tolist() == [flag]
