@@ -408,7 +408,7 @@ size_t spv_verify_sample_workspace_bytes(int32_t B, int32_t gamma, int32_t V);
  * rounding is left (a re-raced draw within a few ulp of another key). */
 #define SPV_FLAG_ACCEPT_BAND 1 /* an examined u lay inside the error band of min(1, p/q) */
 #define SPV_FLAG_DRAW_BAND 2   /* the drawn token's key is within the keys' error bound of another key's */
-#define SPV_FLAG_TOP_P_BAND 4  /* (host) a filtered row's nucleus boundary is within rounding */
+#define SPV_FLAG_TOP_P_BAND 4  /* a filtered row's nucleus boundary is within rounding */
 
 /* One fused verify-sampling step: logits_to_probs (specdec/sampler.py:19-36)
  * on every row, then batch_accept (engine/spec_scheduler.py:46-88) with
@@ -445,6 +445,36 @@ int spv_verify_sample(const float* target, const float* draft, int is_probs,
                       int32_t* new_len, double* accept_prob, int32_t* flags,
                       int32_t decide_only, void* workspace,
                       size_t workspace_bytes, void* stream);
+
+/* The same with top-k / top-p filters (specdec/sampler.py:19-56) on every row
+ * first: logits_to_probs(z, T, top_k, top_p) of the target and draft logits,
+ * T > 0, then the decisions, draw and commit of spv_verify_sample. The filters
+ * are those of spv_filter_logits (top_k <= 0 or >= V, or top_p outside (0, 1):
+ * that filter is off). With 0 < top_k <= 512 one launch keeps each row's
+ * survivors and makes the whole result; sequences it does not cover (a NaN or
+ * infinite logit, more than 1,024 values kept by top-k, a noise entry that is
+ * not above zero), and every other call, take spv_filter_logits' kernel into
+ * target_scratch (B, gamma+1, V) / draft_scratch (B, gamma, V) and then
+ * spv_verify_sample's. flags[b] gets SPV_FLAG_TOP_P_BAND when a value of one
+ * of the sequence's rows lies within rounding of the nucleus edge. The
+ * workspace holds arrival counters that must be zero when it is first used
+ * (zero-filled) and are zero after every call; it is not shared with
+ * spv_verify_sample. */
+size_t spv_verify_sample_filtered_workspace_bytes(int32_t B, int32_t gamma,
+                                                  int32_t V, float temperature,
+                                                  int32_t top_k);
+int spv_verify_sample_filtered(const float* target, const float* draft,
+                               float temperature, int32_t top_k, float top_p,
+                               const int32_t* proposals, const float* u_accept,
+                               const float* exp_noise, const int32_t* start_pos,
+                               const int32_t* remaining, int32_t eos_id,
+                               int32_t B, int32_t gamma, int32_t V,
+                               int32_t* accept_len, int32_t* out_tokens,
+                               int32_t* n_commit, int32_t* finished,
+                               int32_t* new_len, int32_t* flags,
+                               float* target_scratch, float* draft_scratch,
+                               void* workspace, size_t workspace_bytes,
+                               void* stream);
 
 /* One draft step of the draft loop (engine/spec_scheduler.py:243-252): for
  * every row b of the draft logits (row b at logits + b * row_stride, V fp32

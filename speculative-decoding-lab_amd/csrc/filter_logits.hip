@@ -35,7 +35,7 @@
 // sort does not fix that order.
 #include <math.h>
 
-#include "spv_common.h"
+#include "sample_common.h"
 
 using namespace spv;
 
@@ -47,36 +47,21 @@ constexpr int kFThreads = 1024;
 constexpr int kLevels = 3;
 constexpr int kShift[kLevels] = {24, 12, 0}, kLBits[kLevels] = {8, 12, 12}, kLCopies[kLevels] = {16, 1, 1};
 constexpr int kHist = 16 * 257;  // ints (and doubles) of the histogram space: 16 x (256 + 1) >= 4096 + 1
-constexpr float kLog2e = 1.4426950408889634f;
-// Half width of the window around the nucleus edge p W (relative to W) where
-// the reference's fp32 softmax and cumulative sum can keep or drop a value
-// differently from the exact masses: torch's normalisation of a 151,936-entry
-// row is off by up to ~1e-5, and the cumulative sum rounds each entry.
-constexpr double kTopPWindow = 5e-5;
-
-// The fp64 mass exp(x - max) of a key's value, as the histograms sum it.
-__device__ __forceinline__ float key_value(uint32_t k);
-__device__ __forceinline__ double key_mass(uint32_t k, float ml) {
-  return (double)__builtin_amdgcn_exp2f(fmaf(key_value(k), kLog2e, -ml));
-}
-
-// Larger x, larger key; NaN above everything (torch.topk ranks NaN first).
-__device__ __forceinline__ uint32_t order_key(float x) {
-  const uint32_t u = __float_as_uint(x);
-  if (x != x) return 0xffffffffu;
-  return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
-}
-
-__device__ __forceinline__ float key_value(uint32_t k) {
-  return __uint_as_float((k & 0x80000000u) ? (k & 0x7fffffffu) : ~k);
-}
-
-struct FilterArgs {
+// Rows of one or two tensors: row r < rows is row r of the first, the others
+// are row r - rows of the second (a verify step's target and draft rows in one
+// launch: 352 rows of 151,936 fill the CUs that 192 and 160 rows apart leave
+// idle).
+struct FilterTensor {
   const float* in;
   float* out;
   int32_t* ambiguous;  // per row: values whose preceding mass lies within the window of the nucleus edge
+  int per_seq;         // rows per entry of `need`
+};
+struct FilterArgs {
+  FilterTensor t[2];
+  const int32_t* need;  // null, or per sequence: rows of sequences with need == 0 are left alone
   long long in_stride, out_stride;
-  int V, top_k;
+  int rows, V, top_k;
   float tf, top_p;
 };
 
@@ -103,28 +88,6 @@ __device__ __forceinline__ void for_row(const float* z, int V, float tf, F f) {
   for (; i < V; i += kFThreads) f(i, scaled_at<UNIT>(z, i, tf));
 }
 
-// Block-wide exclusive scan of one double per thread (bins in descending order).
-__device__ __forceinline__ double block_exclusive_scan_f64(double v, double* lds, double* total) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  double incl = v;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const double t = __shfl_up(incl, o, 64);
-    if (lane >= o) incl += t;
-  }
-  if (lane == 63) lds[wave] = incl;
-  __syncthreads();
-  double off = 0.0, sum = 0.0;
-  for (int w = 0; w < nw; ++w) {
-    const double x = lds[w];
-    if (w < wave) off += x;
-    sum += x;
-  }
-  __syncthreads();
-  *total = sum;
-  return off + incl - v;
-}
-
 template <bool UNIT>
 __global__ __launch_bounds__(kFThreads) void filter_rows_kernel(FilterArgs a) {
   __shared__ int s_cnt[kHist];
@@ -135,8 +98,13 @@ __global__ __launch_bounds__(kFThreads) void filter_rows_kernel(FilterArgs a) {
   __shared__ int s_digit, s_need, s_tie_lim;
   __shared__ int s_mdigit[3], s_mcabove[3], s_mdcnt[3];
   __shared__ double s_mabove[3], s_tgt[3];
-  const float* z = a.in + (size_t)blockIdx.x * a.in_stride;
-  float* out = a.out + (size_t)blockIdx.x * a.out_stride;
+  const bool second = (int)blockIdx.x >= a.rows;
+  const FilterTensor& ft = a.t[second];
+  const int row = (int)blockIdx.x - (second ? a.rows : 0);
+  if (a.need && !a.need[row / ft.per_seq]) return;
+  const float* z = ft.in + (size_t)row * a.in_stride;
+  float* out = ft.out + (size_t)row * a.out_stride;
+  int32_t* ambiguous = ft.ambiguous;
   const int V = a.V, tid = threadIdx.x;
   const float tf = a.tf;
   const bool do_k = a.top_k > 0 && a.top_k < V;
@@ -326,7 +294,7 @@ __global__ __launch_bounds__(kFThreads) void filter_rows_kernel(FilterArgs a) {
     // searches whose prefixes agree at a level share its pass over the row
     // (the window is narrow, so usually all three do).
     const uint32_t min_key = thr;
-    const int ns = a.ambiguous ? 3 : 1;
+    const int ns = ambiguous ? 3 : 1;
     pmask = 0;
     uint32_t pre[3] = {0u, 0u, 0u};
     double abv[3] = {0.0, 0.0, 0.0};
@@ -364,7 +332,7 @@ __global__ __launch_bounds__(kFThreads) void filter_rows_kernel(FilterArgs a) {
       const double need_c = ceil((s_tgt[0] - above) / wt);
       c = need_c < 1.0 ? 1 : (need_c > (double)total_ties ? total_ties : (long long)need_c);
     }
-    if (a.ambiguous && tid == 0) {
+    if (ambiguous && tid == 0) {
       // Sorted position of the value crossing target t: c_t - 1 ties into its key.
       auto cross_pos = [&](int t) -> long long {
         const double w = key_mass(pre[t], ml);
@@ -379,7 +347,7 @@ __global__ __launch_bounds__(kFThreads) void filter_rows_kernel(FilterArgs a) {
       // after the value crossing the lower edge to the one crossing the upper.
       const long long lo = s_tgt[1] <= 0.0 ? 0 : cross_pos(1) + 1;
       const long long hi = cross_pos(2);
-      a.ambiguous[blockIdx.x] = hi >= lo ? (int)(hi - lo + 1) : 0;
+      ambiguous[row] = hi >= lo ? (int)(hi - lo + 1) : 0;
     }
     thr = tkey;
     if (c < total_ties) {
@@ -404,17 +372,39 @@ __global__ __launch_bounds__(kFThreads) void filter_rows_kernel(FilterArgs a) {
       lim = s_tie_lim;
     }
   }
-  if (a.ambiguous && !do_p && tid == 0) a.ambiguous[blockIdx.x] = 0;
+  if (ambiguous && !do_p && tid == 0) ambiguous[row] = 0;
   for_row<UNIT>(z, V, tf, [&](int i, float x) {
     const uint32_t key = order_key(x);
     out[i] = (key > thr || (key == thr && i <= lim)) ? x : -INFINITY;
   });
 }
 
-// float(max(T, 1e-12)) as the fp32 scalar torch divides by.
-inline float temperature_divisor(float T) { return (float)((double)T > 1e-12 ? (double)T : 1e-12); }
+void launch_filter(const FilterArgs& a, int rows, hipStream_t s) {
+  if (a.tf == 1.0f)
+    hipLaunchKernelGGL(filter_rows_kernel<true>, dim3(rows), dim3(kFThreads), 0, s, a);
+  else
+    hipLaunchKernelGGL(filter_rows_kernel<false>, dim3(rows), dim3(kFThreads), 0, s, a);
+}
 
 }  // namespace
+
+int spv::filter_verify_rows(const float* target, float* target_out, int32_t* amb_t, const float* draft,
+                            float* draft_out, int32_t* amb_d, const int32_t* need, int32_t B, int32_t gamma, int32_t V,
+                            float temperature, int32_t top_k, float top_p, void* stream) {
+  FilterArgs a{};
+  a.t[0] = FilterTensor{target, target_out, amb_t, gamma + 1};
+  a.t[1] = FilterTensor{draft, draft_out, amb_d, gamma};
+  a.need = need;
+  a.in_stride = a.out_stride = V;
+  a.rows = B * (gamma + 1);
+  a.V = V;
+  a.top_k = top_k;
+  a.top_p = top_p;
+  a.tf = temperature_divisor(temperature);
+  launch_filter(a, B * (2 * gamma + 1), (hipStream_t)stream);
+  SPV_CHECK_LAUNCH();
+  return SPV_OK;
+}
 
 extern "C" {
 
@@ -425,19 +415,15 @@ int spv_filter_logits(const float* logits, int64_t in_stride, float* out, int64_
     return SPV_ERR_ARG;
   if (rows == 0) return SPV_OK;
   FilterArgs a{};
-  a.in = logits;
-  a.out = out;
-  a.ambiguous = ambiguous;
+  a.t[0] = FilterTensor{logits, out, ambiguous, 1};
   a.in_stride = in_stride;
   a.out_stride = out_stride;
+  a.rows = rows;
   a.V = V;
   a.top_k = top_k;
   a.top_p = top_p;
   a.tf = temperature_divisor(temperature);
-  if (a.tf == 1.0f)
-    hipLaunchKernelGGL(filter_rows_kernel<true>, dim3(rows), dim3(kFThreads), 0, (hipStream_t)stream, a);
-  else
-    hipLaunchKernelGGL(filter_rows_kernel<false>, dim3(rows), dim3(kFThreads), 0, (hipStream_t)stream, a);
+  launch_filter(a, rows, (hipStream_t)stream);
   SPV_CHECK_LAUNCH();
   return SPV_OK;
 }

@@ -71,6 +71,8 @@ SIGNATURES = {
     "spv_verify_attn_static": (I, [P, P, I, P, P, I, P, P, I, P, P, P, P, I, I, I, I, I, I, I, I, I, F, P]),
     "spv_verify_sample_workspace_bytes": (S, [I, I, I]),
     "spv_verify_sample": (I, [P, P, I, F, P, P, P, P, P, P, I, I, I, I, P, P, P, P, P, P, P, I, P, S, P]),
+    "spv_verify_sample_filtered_workspace_bytes": (S, [I, I, I, F, I]),
+    "spv_verify_sample_filtered": (I, [P, P, F, I, F, P, P, P, P, P, I, I, I, I, P, P, P, P, P, P, P, P, P, S, P]),
     "spv_draft_sample_workspace_bytes": (S, [I, I]),
     "spv_draft_sample": (I, [P, ctypes.c_int64, F, P, I, I, P, I, P, P, P, S, P]),
     "spv_filter_logits": (I, [P, ctypes.c_int64, P, ctypes.c_int64, I, I, F, I, F, P, P]),

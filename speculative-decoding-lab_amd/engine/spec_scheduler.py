@@ -41,6 +41,7 @@ from .attention import VerifyPlan, verify_attention
 from .kv import PagedKVCache, WritePlan
 
 _workspace = _hip.Workspace()
+_filter_workspace = _hip.Workspace()
 _draft_workspace = _hip.Workspace()
 
 
@@ -101,6 +102,24 @@ def _launch_sample(target: torch.Tensor, draft: torch.Tensor, proposals: torch.T
          ptr(r.n_commit) if r else None, ptr(r.finished) if r else None,
          ptr(r.new_len) if r else None, ptr(accept_prob), ptr(flags), 1 if decide_only else 0,
          ptr(ws), int(ws_bytes), _hip.stream_of(dev))
+
+
+def _launch_filtered(target: torch.Tensor, draft: torch.Tensor, proposals: torch.Tensor, u: torch.Tensor,
+                     noise: torch.Tensor, temperature: float, top_k: int, top_p: float,
+                     start_pos: Optional[torch.Tensor], remaining: Optional[torch.Tensor], eos_id: Optional[int],
+                     r: VerifyResult) -> None:
+    B, C, V = (int(x) for x in target.shape)
+    dev = target.device
+    ws_bytes = _hip.lib().spv_verify_sample_filtered_workspace_bytes(B, C - 1, V, temperature, top_k)
+    if ws_bytes == 0:
+        raise ValueError("unsupported verify-sampling shape B={} gamma={} V={}".format(B, C - 1, V))
+    ws = _filter_workspace.get(ws_bytes, dev)
+    # rows of sequences that the one-launch form does not cover are filtered into these
+    ts, ds = torch.empty_like(target), torch.empty_like(draft)
+    call("spv_verify_sample_filtered", ptr(target), ptr(draft), temperature, top_k, top_p, ptr(proposals), ptr(u),
+         ptr(noise), ptr(start_pos), ptr(remaining), -1 if eos_id is None else int(eos_id), B, C - 1, V,
+         ptr(r.accept_len), ptr(r.out_tokens), ptr(r.n_commit), ptr(r.finished), ptr(r.new_len), ptr(r.flags),
+         ptr(ts), ptr(ds), ptr(ws), int(ws_bytes), _hip.stream_of(dev))
 
 
 @dataclass
@@ -181,12 +200,8 @@ def verify_sample(target: torch.Tensor, draft: torch.Tensor, proposals: torch.Te
         raise ValueError("sampling needs the Exp(1) noise rows")
     t = target.float().contiguous()
     d = draft.float().contiguous()
-    amb = None
-    if not greedy and not is_probs and _hip.filtering(top_k, top_p, V):
-        t, amb_t = _hip.filter_rows(t, temperature, top_k, top_p, ambiguous=True)
-        d, amb_d = _hip.filter_rows(d, temperature, top_k, top_p, ambiguous=True)
-        amb = amb_t.sum(1) + amb_d.sum(1)
-        temperature = 1.0
+    filtered = not greedy and not is_probs and _hip.filtering(top_k, top_p, V)
+    if filtered:
         draft_stats = None
     if draft_stats is not None:
         if is_probs or tuple(draft_stats.shape) != (B, gamma, 2) or draft_stats.dtype != torch.float32 \
@@ -201,10 +216,11 @@ def verify_sample(target: torch.Tensor, draft: torch.Tensor, proposals: torch.Te
     rem = None if remaining is None else _hip.i32(remaining, dev)
     if result is None:
         result = _new_result(int(B), int(gamma), dev)
-    _launch_sample(t, d, x, uf, nz, temperature, is_probs, sp, rem, eos_id, False, None, result,
-                   draft_stats=draft_stats)
-    if amb is not None:
-        result.flags.bitwise_or_((amb > 0).to(torch.int32) * _hip.FLAG_TOP_P_BAND)
+    if filtered:
+        _launch_filtered(t, d, x, uf, nz, float(temperature), int(top_k), float(top_p), sp, rem, eos_id, result)
+    else:
+        _launch_sample(t, d, x, uf, nz, temperature, is_probs, sp, rem, eos_id, False, None, result,
+                       draft_stats=draft_stats)
     return result
 
 

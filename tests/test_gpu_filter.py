@@ -186,3 +186,80 @@ def test_draft_sample_with_filters(cuda):
         want = [S.race_argmax(S.logits_to_probs(z[b], 1.0, top_k, top_p), e[b]) for b in range(16)]
         got = es.draft_sample(z.to(cuda), 1.0, e.to(cuda), top_k=top_k, top_p=top_p)
         assert got.tolist() == want, (top_k, top_p)
+
+
+def _general(t, d, x, u, noise, T, top_k, top_p):
+    """Filtered rows, then the unfiltered sampler on them at T = 1."""
+    ft, nt = _hip.filter_rows(t, T, top_k, top_p, ambiguous=True)
+    fd, nd = _hip.filter_rows(d, T, top_k, top_p, ambiguous=True)
+    res = es.verify_sample(ft, fd, x, u, noise, 1.0)
+    res.flags.bitwise_or_(((nt.sum(1) + nd.sum(1)) > 0).int() * _hip.FLAG_TOP_P_BAND)
+    return res
+
+
+@pytest.mark.parametrize("B,gamma,vocab,T,top_k,top_p", [
+    (3, 2, 8, 1.0, 3, 0.7),              # a row shorter than a wave
+    (2, 1, 1023, 0.7, 400, 0.9),         # rows that are not whole float4, few values per thread
+    (3, 4, 50257, 1.3, 50, 0.95),        # the same over several small pieces
+    (1, 32, 10236, 1.0, 20, 1.0),        # one full small piece; the longest draft
+    (1, 3, 10240, 0.5, 512, 0.8),        # one value more than a piece; the largest top_k
+    (40, 5, 40957, 1.0, 100, 0.9),       # two large pieces, unaligned rows
+    (64, 5, 151936, 0.8, 50, 0.9),       # the fused workload
+    (20, 2, 151936, 1.0, 513, 0.9),      # top_k above the short form's
+])
+def test_filtered_sampler_short_form_equals_the_general_path(cuda, B, gamma, vocab, T, top_k, top_p):
+    g = torch.Generator(device=cuda).manual_seed(B * 1000 + vocab)
+    t = torch.randn(B, gamma + 1, vocab, generator=g, device=cuda) * 2
+    d = t[:, :gamma] + 0.5 * torch.randn(B, gamma, vocab, generator=g, device=cuda)
+    # bf16-valued rows (ties at the edges), rows with most entries masked, values of both signs of zero
+    t[0] = t[0].bfloat16().float()
+    if B > 1:
+        t[1, 0, 5:] = float("-inf")
+        d[1, 0, 5:] = float("-inf")
+        t[1, 1] = torch.where(t[1, 1] > 0, 0.0, -0.0)
+    d = d.contiguous()
+    q = torch.softmax(_hip.filter_rows(d, T, top_k, top_p), -1)
+    x = torch.multinomial(q.reshape(-1, vocab), 1, generator=g).reshape(B, gamma).int()
+    u = torch.rand(B, gamma, generator=g, device=cuda)
+    noise = torch.empty(B, vocab, device=cuda).exponential_(1, generator=g)
+    want = _general(t, d, x, u, noise, T, top_k, top_p)
+    for _ in range(2):  # the arrival counters are left at zero
+        got = es.verify_sample(t, d, x, u, noise, T, top_k=top_k, top_p=top_p)
+        certain = (want.flags | got.flags) == 0
+        assert torch.equal(got.accept_len[certain], want.accept_len[certain])
+        assert torch.equal(got.out_tokens[certain], want.out_tokens[certain])
+        assert torch.equal(got.n_commit, got.accept_len + 1)
+        differ = int(((got.out_tokens != want.out_tokens).any(1)).sum())
+        assert differ <= B // 16, differ  # flagged sequences mostly agree as well
+        # the nucleus window's count moves only where a value lies at the window's own rim
+        assert int((got.flags != want.flags).sum()) <= B // 16 + (1 if top_p < 1 else 0)
+
+
+@pytest.mark.parametrize("odd", ["nan", "inf", "ties", "masked", "zero_noise", "tiny_T"])
+def test_filtered_sampler_rows_the_short_form_leaves(cuda, odd):
+    """Sequence 1's rows or noise are outside the short form; the others' are not."""
+    B, gamma, vocab, T = 4, 3, 30000, 1.0
+    g = torch.Generator(device=cuda).manual_seed(3)
+    t = torch.randn(B, gamma + 1, vocab, generator=g, device=cuda) * 2
+    d = t[:, :gamma] + torch.randn(B, gamma, vocab, generator=g, device=cuda)
+    noise = torch.empty(B, vocab, device=cuda).exponential_(1, generator=g)
+    if odd == "nan":
+        t[1, 0, 77] = float("nan")
+    elif odd == "inf":
+        d[1, 1, 4000] = float("inf")
+    elif odd == "ties":
+        t[1, 0] = 1.0  # every value is the k-th largest
+    elif odd == "masked":
+        t[1, 2] = float("-inf")
+    elif odd == "zero_noise":
+        noise[1, 12345] = 0.0
+    else:
+        T = 1e-4  # the whole call
+    d = d.contiguous()
+    x = d.nan_to_num(0.0, 0.0).argmax(-1).int()
+    u = torch.rand(B, gamma, generator=g, device=cuda)
+    want = _general(t, d, x, u, noise, T, 40, 0.9)
+    got = es.verify_sample(t, d, x, u, noise, T, top_k=40, top_p=0.9)
+    assert torch.equal(got.accept_len, want.accept_len)
+    assert torch.equal(got.out_tokens, want.out_tokens)
+    assert torch.equal(got.flags, want.flags)
