@@ -22,9 +22,13 @@
 // P^T's layout is exactly the accumulator layout of S^T (lane l holds keys
 // 4*(l/16)+0..3 of query column l%16), so the online-softmax rescale stays
 // inside a lane; the row max needs two cross-lane steps (xor 16, 32).
+// fp32 queries over fp32 pages (same shapes) take the same walk on
+// v_mfma_f32_16x16x4_f32.
 // VALU path: any dtype / head_dim <= 256 / block size, fp32 math with LDS tiles,
 // a (sequence, kv head, row group, split) grid and its own merge kernel.
 #include <math.h>
+
+#include <type_traits>
 
 #include <hip/hip_ext.h>
 
@@ -264,7 +268,9 @@ __host__ __device__ constexpr int ring_depth(int, int, int) { return 2; }
 // head_dim 128; measured best among 24..56 at batch 128, 16/2 heads, contexts
 // log-uniform in [512, 8192], 2-3% ahead of 48, the best before the combine
 // and spill fixes), scaled to the page size.
-__host__ __device__ constexpr int piece_cost(int d, int kt) { return 32 * 8192 / (16 * d * 2 * (kt == SPV_FP8E4M3 ? 1 : 2)); }
+__host__ __device__ constexpr int piece_cost(int d, int kt) { 
+  return 32 * 8192 / (16 * d * 2 * (kt == SPV_FP8E4M3 ? 1 : kt == SPV_F32 ? 4 : 2));
+}
 constexpr int kMfmaThreads = 512;
 // The smallest piece of the equal-pieces split, in pages, for a longest
 // context of `maxnp` pages: cutting finer than fills the workgroups' waves
@@ -579,6 +585,11 @@ struct PageRegs<D, SPV_BF16> {
 template <int D>
 struct PageRegs<D, SPV_F16> : PageRegs<D, SPV_BF16> {};
 template <int D>
+struct PageRegs<D, SPV_F32> {
+  uint4 k[D / 16];  // key i16, dims 16 ks + 4 g .. + 3
+  uint4 v[D / 16];  // dim 16 mt + i16, keys 4 g .. 4 g + 3
+};
+template <int D>
 struct PageRegs<D, SPV_FP8E4M3> {
   uint2 k[D / 32];     // key i16, dims 32 ks + 8 g .. + 7 (codes)
   uint32_t v[D / 16];  // dim 16 mt + i16, keys 4 g .. 4 g + 3 (codes)
@@ -690,8 +701,7 @@ __device__ void merge_segment(const AttnParams& p, SlotOf slot_of, int ns, int b
       *reinterpret_cast<uint2*>(static_cast<uint16_t*>(p.out) + ob) =
           pack4_out<QT>(acc[it][0] * inv, acc[it][1] * inv, acc[it][2] * inv, acc[it][3] * inv);
     } else {
-#pragma unroll
-      for (int k = 0; k < 4; ++k) store_out<QT>(p, ob + k, acc[it][k] * inv);
+      *reinterpret_cast<f32x4_t*>(static_cast<float*>(p.out) + ob) = acc[it] * inv;
     }
   }
 }
@@ -712,22 +722,34 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void attn_mfma_kernel(AttnParams p
   // fp16 pages take fp16 queries (S^T and P V on the fp16 MFMAs); bf16 and
   // fp8 pages take bf16 queries.
   constexpr bool kF16 = KT == SPV_F16;
-  static_assert(QT == (kF16 ? SPV_F16 : SPV_BF16), "query type follows the page type");
+  // fp32 pages take fp32 queries: S^T and P V on v_mfma_f32_16x16x4_f32, fp32
+  // operands and sums throughout. The order of a k-step's keys and dims is
+  // free as long as both operands share it: lane group g of step jj holds dim
+  // 16 ks + 4 g + jj (S^T) or key 4 g + jj (P V), so K, V^T and the queries
+  // come in 16-byte pieces and P^T is S^T's accumulator as it stands. The VALU
+  // kernel these calls took is bound by its serial 16-key tiles (one element per
+  // load, bank-conflicting LDS reads, four barriers a tile): 4 sequences of 37 to
+  // 129 keys, chunk 5, 4/2 heads of 64, kernels of a call 86 us; a whole list call
+  // (write, attend, rewind) 276 -> 202 us, error against float64 2.7e-7 -> 2.2e-7.
+  constexpr bool kF32 = KT == SPV_F32;
+  static_assert(QT == (kF32 ? SPV_F32 : kF16 ? SPV_F16 : SPV_BF16), "query type follows the page type");
+  using QE = std::conditional_t<kF32, float, uint16_t>;
+  constexpr int kQV = 16 / (int)sizeof(QE);  // query elements in 16 bytes
   // Block ids (and fp8 scales) of a window per lane, or per page from LDS
   // (see the page walk).
-  constexpr bool kLaneIds = D == 64 || NT <= 2 || (NT == 3 && PL);
+  constexpr bool kLaneIds = D == 64 || (NT <= 2 && !(kF32 && NT == 2)) || (NT == 3 && PL);
   constexpr int KS = D / 32;  // 32-dim k-steps of S^T
   constexpr int MT = D / 16;  // 16-dim tiles of O^T
   constexpr int BS = 16;
   constexpr int RPG = 16 * NT;
   constexpr int NWV = kMfmaThreads / 64;
-  constexpr int QSTR = D + 8;  // bf16 row stride of the staged queries
+  constexpr int QSTR = D + kQV;  // element stride of the staged query rows
   extern __shared__ int s_pref[];
   // The staged query rows (page walk) and the combine slots (after it) share LDS.
   constexpr int TPR = combine_tiles(NT, MT);  // O^T tiles combined per round
-  constexpr int kQBytes = RPG * QSTR * 2, kXBytes = NWV * RPG * 16 * TPR * 4;
+  constexpr int kQBytes = RPG * QSTR * (int)sizeof(QE), kXBytes = NWV * RPG * 16 * TPR * 4;
   __shared__ __align__(16) char s_union[kQBytes > kXBytes ? kQBytes : kXBytes];
-  uint16_t* sQ = reinterpret_cast<uint16_t*>(s_union);
+  QE* sQ = reinterpret_cast<QE*>(s_union);
   float* sm_x = reinterpret_cast<float*>(s_union);  // [wave][tile of the round][row][16 dims]
   // Block ids of the pages being walked. Reading them from LDS keeps the page
   // loads in flight: a vector load of a table entry would need vmcnt(0), which
@@ -798,11 +820,11 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void attn_mfma_kernel(AttnParams p
     T = r.T;
   }
   auto page_start = [&](long long w) { return div_floor(w * T, nw); };
-  const uint16_t* kbase = static_cast<const uint16_t*>(p.kpool);
-  const uint16_t* vbase = static_cast<const uint16_t*>(p.vpool);
+  const QE* kbase = static_cast<const QE*>(p.kpool);
+  const QE* vbase = static_cast<const QE*>(p.vpool);
   const uint8_t* kbase8 = static_cast<const uint8_t*>(p.kpool);
   const uint8_t* vbase8 = static_cast<const uint8_t*>(p.vpool);
-  const uint16_t* qbase = static_cast<const uint16_t*>(p.q);
+  const QE* qbase = static_cast<const QE*>(p.q);
   const float sl2 = p.scale_log2;
 
   // The share's units left, 32-bit (a share holds far fewer than 2^31): with
@@ -853,6 +875,13 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void attn_mfma_kernel(AttnParams p
           f.sk = sc.x;
           f.sv = sc.y;
         }
+      } else if constexpr (kF32) {
+        const float* kp = kbase + slot;
+        const float* vp = vbase + slot;
+#pragma unroll
+        for (int ks = 0; ks < D / 16; ++ks) f.k[ks] = *reinterpret_cast<const uint4*>(kp + i16 * D + 16 * ks + 4 * g);
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) f.v[mt] = *reinterpret_cast<const uint4*>(vp + (16 * mt + i16) * BS + 4 * g);
       } else if constexpr (NT >= 4) {
         const __amdgpu_buffer_rsrc_t rk = span_rsrc(kbase + slot, BS * D * 2);
         const __amdgpu_buffer_rsrc_t rv = span_rsrc(vbase + slot, BS * D * 2);
@@ -867,8 +896,8 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void attn_mfma_kernel(AttnParams p
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) f.v[mt] = __builtin_bit_cast(uint2, load_b64(rv, lv, 32u * BS * mt));
       } else {
-        const uint16_t* kp = kbase + slot;
-        const uint16_t* vp = vbase + slot;
+        const QE* kp = kbase + slot;
+        const QE* vp = vbase + slot;
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) f.k[ks] = *reinterpret_cast<const uint4*>(kp + i16 * D + 32 * ks + 8 * g);
 #pragma unroll
@@ -912,10 +941,10 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void attn_mfma_kernel(AttnParams p
     // at head_dim 128: 88 -> 87 us per layer at batch 128, Qwen2.5-3B heads).
     // The head_dim-128 kernels with three query tiles in the cost-balanced
     // split keep the item-by-item loop: the batch's registers make them spill.
-    constexpr bool kBatchStage = D == 64 || NT <= 2 || NT == 4 || (NT == 3 && !BAL);
+    constexpr bool kBatchStage = D == 64 || kF32 || NT <= 2 || NT == 4 || (NT == 3 && !BAL);
     if constexpr (kBatchStage) {
       static_assert(kTabChunk == kMfmaThreads, "one block id per thread");
-      constexpr int kQItems = (RPG * (D / 8) + kMfmaThreads - 1) / kMfmaThreads;
+      constexpr int kQItems = (RPG * (D / kQV) + kMfmaThreads - 1) / kMfmaThreads;
       // The thread index is opaque so that no staging address is hoisted out
       // of the piece loop, where it would live across the walk.
       int stid = threadIdx.x;
@@ -928,11 +957,11 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void attn_mfma_kernel(AttnParams p
 #pragma unroll
       for (int k = 0; k < kQItems; ++k) {
         const int idx = stid + k * kMfmaThreads;
-        const int rr = idx / (D / 8), c = idx - rr * (D / 8);
+        const int rr = idx / (D / kQV), c = idx - rr * (D / kQV);
         qv[k] = make_uint4(0, 0, 0, 0);
         if (rr < nr) {  // rr < nr <= RPG: idx is in range
           const int r = qr0 + rr, j = r / p.ratio, hq = h * p.ratio + (r - j * p.ratio);
-          qv[k] = *reinterpret_cast<const uint4*>(qbase + (((size_t)b * p.C + j) * p.Hq + hq) * D + 8 * c);
+          qv[k] = *reinterpret_cast<const uint4*>(qbase + (((size_t)b * p.C + j) * p.Hq + hq) * D + kQV * c);
         }
       }
       // Issued after the staging loads, so their wait does not include it.
@@ -943,8 +972,8 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void attn_mfma_kernel(AttnParams p
 #pragma unroll
       for (int k = 0; k < kQItems; ++k) {
         const int idx = stid + k * kMfmaThreads;
-        const int rr = idx / (D / 8), c = idx - rr * (D / 8);
-        if (idx < RPG * (D / 8)) *reinterpret_cast<uint4*>(&sQ[rr * QSTR + 8 * c]) = qv[k];
+        const int rr = idx / (D / kQV), c = idx - rr * (D / kQV);
+        if (idx < RPG * (D / kQV)) *reinterpret_cast<uint4*>(&sQ[rr * QSTR + kQV * c]) = qv[k];
       }
     } else {
       const int lenv = !PL && threadIdx.x == 0 && p.lens ? p.lens[sid] : 0x7fffffff;
@@ -953,14 +982,14 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void attn_mfma_kernel(AttnParams p
       for (int t = threadIdx.x; t < min(kTabChunk, lp1 - lp0); t += blockDim.x)
         sTab[t] = safe_block(p, table[lp0 + t], b);
       if (lenv < L) flag_bad_read(p, b);
-      for (int idx = threadIdx.x; idx < RPG * (D / 8); idx += blockDim.x) {
-        const int rr = idx / (D / 8), c = idx - rr * (D / 8);
+      for (int idx = threadIdx.x; idx < RPG * (D / kQV); idx += blockDim.x) {
+        const int rr = idx / (D / kQV), c = idx - rr * (D / kQV);
         uint4 v = make_uint4(0, 0, 0, 0);
         if (rr < nr) {
           const int r = qr0 + rr, j = r / p.ratio, hq = h * p.ratio + (r - j * p.ratio);
-          v = *reinterpret_cast<const uint4*>(qbase + (((size_t)b * p.C + j) * p.Hq + hq) * D + 8 * c);
+          v = *reinterpret_cast<const uint4*>(qbase + (((size_t)b * p.C + j) * p.Hq + hq) * D + kQV * c);
         }
-        *reinterpret_cast<uint4*>(&sQ[rr * QSTR + 8 * c]) = v;
+        *reinterpret_cast<uint4*>(&sQ[rr * QSTR + kQV * c]) = v;
       }
     }
     __syncthreads();
@@ -981,7 +1010,7 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void attn_mfma_kernel(AttnParams p
     // which then bounds the walk (fp8 pages most). There the query fragments
     // stay in registers for the whole walk, and the softmax takes the lean
     // form of compute_page. (At head_dim 128 both measured slower.)
-    constexpr bool kLean = D == 64;
+    constexpr bool kLean = D == 64 && !kF32;
     uint4 qreg[kLean ? KS : 1][kLean ? NT : 1];
     if constexpr (kLean) {
 #pragma unroll
@@ -1023,7 +1052,7 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void attn_mfma_kernel(AttnParams p
       // V^T as 16-bit values: the page registers themselves, or an fp8 page's
       // conversion (fp16 or bf16, as above).
       uint2 vb8[kFp8 ? MT : 1];
-      auto vfrag = [&](int mt) -> uint2& {
+      auto vfrag = [&](int mt) -> auto& {
         if constexpr (kFp8) return vb8[mt];
         else return f.v[mt];
       };
@@ -1041,12 +1070,20 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void attn_mfma_kernel(AttnParams p
         // Keys at or beyond L are stale pool contents: zero their V.
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
+          if constexpr (kF32) {
+            if (kpos0 + 0 >= L) f.v[mt].x = 0u;
+            if (kpos0 + 1 >= L) f.v[mt].y = 0u;
+            if (kpos0 + 2 >= L) f.v[mt].z = 0u;
+            if (kpos0 + 3 >= L) f.v[mt].w = 0u;
+            continue;
+          } else {
           uint32_t lo = vfrag(mt).x, hi = vfrag(mt).y;
           if (kpos0 + 0 >= L) lo &= 0xffff0000u;
           if (kpos0 + 1 >= L) lo &= 0x0000ffffu;
           if (kpos0 + 2 >= L) hi &= 0xffff0000u;
           if (kpos0 + 3 >= L) hi &= 0x0000ffffu;
           vfrag(mt) = make_uint2(lo, hi);
+          }
         }
       }
       // An fp8 page's K scale multiplies its scores, its V scale the P that
@@ -1063,6 +1100,18 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void attn_mfma_kernel(AttnParams p
       f32x4_t sc[NT];
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) sc[nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      if constexpr (kF32) {
+#pragma unroll
+        for (int ks = 0; ks < D / 16; ++ks)
+#pragma unroll
+          for (int nt = 0; nt < NT; ++nt) {
+            const f32x4_t qv = *reinterpret_cast<const f32x4_t*>(&sQ[(16 * nt + i16) * QSTR + 16 * ks + 4 * g]);
+            const f32x4_t kv = __builtin_bit_cast(f32x4_t, f.k[ks]);
+#pragma unroll
+            for (int jj = 0; jj < 4; ++jj)
+              sc[nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[jj], qv[jj], sc[nt], 0, 0, 0);
+          }
+      } else {
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
@@ -1077,6 +1126,7 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void attn_mfma_kernel(AttnParams p
             sc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, k_frag<D>(f, ks)),
                                                              __builtin_bit_cast(bf16x8_t, qv), sc[nt], 0, 0, 0);
         }
+      }
       const bool need_mask = page * BS + BS - 1 > start;
       float x[NT][4];
       bool grow = false;
@@ -1183,7 +1233,20 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void attn_mfma_kernel(AttnParams p
           }
         }
       };
-      if constexpr (h16) {
+      if constexpr (kF32) {
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+          float e[4];
+          p_tile(nt, e);
+#pragma unroll
+          for (int mt = 0; mt < MT; ++mt) {
+            const f32x4_t vv = __builtin_bit_cast(f32x4_t, f.v[mt]);
+#pragma unroll
+            for (int jj = 0; jj < 4; ++jj)
+              o[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[jj], e[jj], o[mt][nt], 0, 0, 0);
+          }
+        }
+      } else if constexpr (h16) {
         const float o_down = __builtin_bit_cast(float, (uint32_t)(127 - vc) << 23);
         if (vc) {
 #pragma unroll
@@ -1404,8 +1467,7 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void attn_mfma_kernel(AttnParams p
             *reinterpret_cast<uint2*>(static_cast<uint16_t*>(p.out) + cbase[ci] + e0) =
                 pack4_out<QT>(acc[0] * cinv, acc[1] * cinv, acc[2] * cinv, acc[3] * cinv);
           } else {
-#pragma unroll
-            for (int k = 0; k < 4; ++k) store_out<QT>(p, cbase[ci] + e0 + k, acc[k] * cinv);
+            *reinterpret_cast<f32x4_t*>(static_cast<float*>(p.out) + cbase[ci] + e0) = acc * cinv;
           }
         } else {
           store4_coherent(ro, (size_t)(cbase[ci] + e0) * sizeof(float), acc);
@@ -1546,11 +1608,20 @@ struct Plan {
   // 128 kernels with four query tiles have no registers to spare: the planned
   // prologue made them spill in the page walk (the batch-128 Qwen2.5-3B shape
   // ran 90.8 -> 97.5 us per layer), so they keep the in-kernel prologue.
-  bool plannable() const { return mfma && !(nt == 4 && rows_per_group == 64 && d128); }
-  bool d128;
+  // fp32 pages have no planned kernels either (the parity engine's list calls
+  // make no plan).
+  bool plannable() const { return mfma && !f32 && !(nt == 4 && rows_per_group == 64 && d128); }
+  bool d128, f32;
 };
 
-Plan make_plan(int B, int C, int Hq, int Hkv, int d, int bs, int max_ctx, int kv_dtype, int q_dtype) {
+// Query tiles per row group of the fp32 kernels: an fp32 page takes twice the
+// registers of a 16-bit one, and two pages, O^T and the scores fit the 256 of a
+// wave without scratch up to here.
+constexpr int f32_tiles(int d) { return d == 128 ? 2 : 4; }
+
+// `valu`: the VALU path's plan, whatever the shape and types.
+Plan make_plan(int B, int C, int Hq, int Hkv, int d, int bs, int max_ctx, int kv_dtype, int q_dtype,
+               bool valu = false) {
   Plan pl{};
   const int G = C * (Hq / Hkv);
   // The MFMA kernel addresses the output and the partial slots with 32-bit
@@ -1559,13 +1630,15 @@ Plan make_plan(int B, int C, int Hq, int Hkv, int d, int bs, int max_ctx, int kv
                       2LL * kMfmaWGsMax * G * d * (long long)sizeof(float) < (1LL << 31);
   // Any G: below 16 rows (decode, G = Hq / Hkv) the one query tile is padded
   // with zero rows; the pages still cross HBM once, which is what bounds it.
-  pl.mfma = (((kv_dtype == SPV_BF16 || kv_dtype == SPV_FP8E4M3) && q_dtype == SPV_BF16) ||
+  pl.f32 = kv_dtype == SPV_F32 && q_dtype == SPV_F32;
+  pl.mfma = !valu && (pl.f32 || ((kv_dtype == SPV_BF16 || kv_dtype == SPV_FP8E4M3) && q_dtype == SPV_BF16) ||
              (kv_dtype == SPV_F16 && q_dtype == SPV_F16)) && bs == 16 &&
             (d == 128 || d == 64) && B <= kMfmaMaxB && fits32;
   const int max_pages = (max_ctx + bs - 1) / bs;
   pl.d128 = d == 128;
   if (pl.mfma) {
     pl.nt = G >= 64 ? 4 : (G + 15) / 16;
+    if (pl.f32) pl.nt = min(pl.nt, f32_tiles(d));
     pl.rows_per_group = 16 * pl.nt;
     pl.nrg = (G + pl.rows_per_group - 1) / pl.rows_per_group;
     // One arrival counter per segment.
@@ -1688,6 +1761,29 @@ void launch_mfma(const AttnParams& p, int nt, hipStream_t s) {
   }
 }
 
+// fp32 pages: unplanned calls, query tiles up to f32_tiles(D).
+template <int D, bool BAL>
+void launch_mfma_f32_mode(const AttnParams& p, int nt, hipStream_t s, dim3 grid, size_t smem) {
+  const dim3 blk(kMfmaThreads);
+  switch (nt) {
+    case 1: launch_attn(attn_mfma_kernel<1, D, SPV_F32, BAL, SPV_F32, false>, grid, blk, smem, s, true, true, p); break;
+    case 2: launch_attn(attn_mfma_kernel<2, D, SPV_F32, BAL, SPV_F32, false>, grid, blk, smem, s, true, true, p); break;
+    default:
+      if constexpr (f32_tiles(D) > 2) {
+        if (nt == 3) launch_attn(attn_mfma_kernel<3, D, SPV_F32, BAL, SPV_F32, false>, grid, blk, smem, s, true, true, p);
+        else launch_attn(attn_mfma_kernel<4, D, SPV_F32, BAL, SPV_F32, false>, grid, blk, smem, s, true, true, p);
+      }
+      break;
+  }
+}
+template <int D>
+void launch_mfma_f32(const AttnParams& p, int nt, hipStream_t s) {
+  const size_t smem = (size_t)4 * (p.B + 1) * sizeof(int);
+  const int nw = persistent_wgs();
+  if (balanced_split(p, nw)) launch_mfma_f32_mode<D, true>(p, nt, s, dim3(nw), smem);
+  else launch_mfma_f32_mode<D, false>(p, nt, s, dim3(nw), smem);
+}
+
 void launch_plan(const AttnParams& p, int d, int kv_dtype, hipStream_t s) {
   const size_t smem = (size_t)4 * (p.B + 1) * sizeof(int);
   const int nw = persistent_wgs();
@@ -1706,7 +1802,7 @@ size_t spv_verify_attn_workspace_bytes(int32_t B, int32_t C, int32_t num_q_heads
     return 0;
   // The plan depends on dtypes only through the MFMA choice; size for the larger one.
   const Plan a = make_plan(B, C, num_q_heads, num_kv_heads, head_dim, block_size, max_ctx, SPV_BF16, SPV_BF16);
-  const Plan v = make_plan(B, C, num_q_heads, num_kv_heads, head_dim, block_size, max_ctx, SPV_F32, SPV_F32);
+  const Plan v = make_plan(B, C, num_q_heads, num_kv_heads, head_dim, block_size, max_ctx, SPV_F32, SPV_F32, true);
   const size_t wa = workspace_for(a, B, C, num_q_heads, num_kv_heads, head_dim);
   const size_t wv = workspace_for(v, B, C, num_q_heads, num_kv_heads, head_dim);
   return wa > wv ? wa : wv;
@@ -1735,9 +1831,22 @@ int spv::verify_attn_impl(void* out, const void* q, int q_dtype, const void* k_p
       capacity < 1 || max_ctx < C || max_blocks_per_seq < (max_ctx + block_size - 1) / block_size)
     return SPV_ERR_ARG;
   if (B == 0) return SPV_OK;
-  const Plan pl = make_plan(B, C, num_q_heads, num_kv_heads, head_dim, block_size, max_ctx, kv_dtype, q_dtype);
+  Plan pl = make_plan(B, C, num_q_heads, num_kv_heads, head_dim, block_size, max_ctx, kv_dtype, q_dtype);
   const int nw_layout = exact_layout ? persistent_wgs() : kMfmaWGsMax;
-  const size_t need = workspace_for(pl, B, C, num_q_heads, num_kv_heads, head_dim, nw_layout);
+  size_t need = workspace_for(pl, B, C, num_q_heads, num_kv_heads, head_dim, nw_layout);
+  // fp32 calls are held to the VALU path's workspace (what an allocation-free
+  // caller may rely on being accepted or refused by), and take it when the
+  // workspace is smaller than the MFMA kernels' partial slots: that path needs
+  // less for short contexts and none for the shortest.
+  if (pl.mfma && pl.f32) {
+    const Plan v = make_plan(B, C, num_q_heads, num_kv_heads, head_dim, block_size, max_ctx, kv_dtype, q_dtype, true);
+    const size_t vneed = workspace_for(v, B, C, num_q_heads, num_kv_heads, head_dim, nw_layout);
+    if (vneed > 0 && (!workspace || workspace_bytes < vneed)) return SPV_ERR_WORKSPACE;
+    if (!workspace || workspace_bytes < need) {
+      pl = v;
+      need = vneed;
+    }
+  }
   if (need > 0 && (!workspace || workspace_bytes < need)) return SPV_ERR_WORKSPACE;
 
   AttnParams p{};
@@ -1781,6 +1890,7 @@ int spv::verify_attn_impl(void* out, const void* q, int q_dtype, const void* k_p
   if (pl.mfma) {
     switch (kv_dtype) {
       case SPV_FP8E4M3: head_dim == 128 ? launch_mfma<128, SPV_FP8E4M3>(p, pl.nt, s) : launch_mfma<64, SPV_FP8E4M3>(p, pl.nt, s); break;
+      case SPV_F32: head_dim == 128 ? launch_mfma_f32<128>(p, pl.nt, s) : launch_mfma_f32<64>(p, pl.nt, s); break;
       case SPV_F16: head_dim == 128 ? launch_mfma<128, SPV_F16>(p, pl.nt, s) : launch_mfma<64, SPV_F16>(p, pl.nt, s); break;
       default: head_dim == 128 ? launch_mfma<128, SPV_BF16>(p, pl.nt, s) : launch_mfma<64, SPV_BF16>(p, pl.nt, s); break;
     }
