@@ -342,6 +342,22 @@ int spv_verify_attn_planned(void* out, const void* q, int q_dtype,
                             const void* plan, void* workspace,
                             size_t workspace_bytes, void* stream);
 
+/* spv_kv_write_planned of a later layer's chunk, then spv_verify_attn_planned
+ * over it (the write-then-attend order of engine/model.py:182-190), in one
+ * launch where the planned kernels run over bf16 or fp16 pages: k_new / v_new
+ * (B, C, Hkv, d) in kv_dtype go to the rows of write_plan first. Arguments and
+ * limits are those of the two calls; k_new / v_new must not overlap out. */
+int spv_verify_attn_append_planned(void* out, const void* q, int q_dtype,
+                                   void* k_pool, void* v_pool, int kv_dtype,
+                                   const int32_t* block_tables, int32_t max_blocks_per_seq,
+                                   const int32_t* seq_ids, const int32_t* start_pos,
+                                   const int32_t* seq_lens, int32_t* ctr,
+                                   int32_t B, int32_t C, int32_t num_q_heads, int32_t num_kv_heads,
+                                   int32_t head_dim, int32_t block_size, int32_t layer,
+                                   int32_t capacity, int32_t max_ctx, float scale, const void* plan,
+                                   const void* k_new, const void* v_new, const int32_t* write_plan,
+                                   void* workspace, size_t workspace_bytes, void* stream);
+
 /* spv_verify_attn with no allocation and no caller workspace. No counterpart
  * in the reference: it serves callers that cannot allocate device memory
  * (code under HIP graph capture, tight serving loops, harnesses that forbid

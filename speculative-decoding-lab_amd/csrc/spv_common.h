@@ -192,13 +192,15 @@ __device__ __forceinline__ bool arrive_last(int* counter, int total, int* s_flag
   return *s_flag;
 }
 
-// spv_verify_attn with the workspace passed in (verify_attn.hip).
+// spv_verify_attn with the workspace passed in (verify_attn.hip). `k_new`,
+// `v_new`, `write_plan`: the chunk of spv_verify_attn_append_planned, or null.
 int verify_attn_impl(void* out, const void* q, int q_dtype, const void* k_pool, const void* v_pool, int kv_dtype,
                      const float* kv_scales, const int32_t* block_tables, int32_t max_blocks_per_seq,
                      const int32_t* seq_ids, const int32_t* start_pos, const int32_t* seq_lens, int32_t* ctr,
                      int32_t B, int32_t C, int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim,
                      int32_t block_size, int32_t layer, int32_t capacity, int32_t max_ctx, float scale,
-                     const void* plan, void* workspace, size_t workspace_bytes, bool exact_layout, void* stream);
+                     const void* plan, void* workspace, size_t workspace_bytes, bool exact_layout, void* stream,
+                     const void* k_new = nullptr, const void* v_new = nullptr, const int32_t* write_plan = nullptr);
 
 }  // namespace spv
 

@@ -72,6 +72,12 @@ struct AttnParams {
   int max_pages;     // ceil(max_ctx / block_size): no table entry beyond it is read
   float scale_log2;  // softmax scale * log2(e)
   int* plan;         // MFMA path: the round's plan (written by attn_plan_kernel, read by planned calls)
+  // Planned calls over 16-bit pages: this layer's chunk (B, C, Hkv, d) and the
+  // pool row of each of its tokens, to be written before it is attended
+  // (knew NULL: the chunk is in the pool already).
+  const void* knew;
+  const void* vnew;
+  const int32_t* wplan;
 };
 
 // Pages of sequence b's context, never more than the caller-declared bound.
@@ -716,7 +722,8 @@ __device__ __forceinline__ int xswz(int r) { return ((r >> 1) ^ (r >> 3)) & 3; }
 // PL: the call reads the round's plan (attn_plan_kernel) instead of making
 // it: its first piece and the block ids of each wave's first page come in one
 // load, so the page walk starts one round trip after launch.
-template <int NT, int D, int QT, bool BAL, int KT, bool PL>
+// AP: a planned call that writes its chunk's keys and values first.
+template <int NT, int D, int QT, bool BAL, int KT, bool PL, bool AP = false>
 __global__ __launch_bounds__(kMfmaThreads, 1) void attn_mfma_kernel(AttnParams p) {
   constexpr bool kFp8 = KT == SPV_FP8E4M3;
   // fp16 pages take fp16 queries (S^T and P V on the fp16 MFMAs); bf16 and
@@ -910,6 +917,110 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void attn_mfma_kernel(AttnParams p
     PageRegs<D, KT> buf[kRing];
 
 
+    // A call given the chunk (AP) writes it: the wave that walks a
+    // page first stores the chunk's tokens in it (write-then-attend,
+    // engine/model.py:182-190), so its own later loads of the page see them with
+    // no barrier and no wait (a wave's vector memory operations reach its CU's
+    // cache in order); waves of the other row groups of the kv head write the
+    // same bytes for themselves, and the last piece of a segment takes the
+    // tokens past max_ctx too. The new rows are loaded with the queries and
+    // stored behind the loads of the wave's first page (unless that page is the
+    // chunk's), in the time the queries take to arrive. A launch of
+    // its own for the write took 4.0-4.9 us per layer, nearly all of it launch
+    // and one round trip; in here it adds 1.3-3 us (28 layers of 8 sequences of 64
+    // to 1,024 keys, 12/2 heads of 128, a whole round 702 -> 632 us; two draft
+    // steps of 24 layers, 32 sequences, 14/2 heads of 64, 824 -> 737; with the
+    // rows loaded and stored before the first page 764).
+    constexpr bool kAppend = AP;
+    // (head_dim 128 with three query tiles: its rows are loaded after the first
+    // page; in flight beside it they made the walk spill)
+    constexpr bool kLate = !(NT == 3 && D == 128);
+    constexpr int kTok = 8;                                                  // tokens per batch of loads
+    constexpr int kVec = D * 2 / 16, kTP = 64 / kVec, kKI = kTok / kTP;      // 16-byte pieces of a key
+    constexpr int kTV = 128 / D, kVI = kTok / kTV;                           // a value row as D / 2 pairs
+    bool own = false, pre = first;  // this wave stores a page's tokens; its first page is loaded early
+    int cpg = 0, ca = 0, cb = 0;    // that page, and the chunk tokens in it
+    int32_t adst = -1;
+    u32x4_t akq[kAppend ? kKI : 1];
+    uint32_t avq[kAppend ? kVI : 1];
+    // (the lane from an opaque thread index: nothing of this lives across the walk)
+    auto opaque_lane = [&]() {
+      int t = threadIdx.x;
+      asm volatile("" : "+v"(t));
+      return t & 63;
+    };
+    auto append_load = [&](int j0) {  // tokens j0 .. min(j0 + kTok, cb) - 1
+      const int al = opaque_lane(), nj = min(kTok, cb - j0);
+      const size_t tstride = (size_t)p.Hkv * D;
+      const size_t src = ((size_t)b * p.C + j0) * tstride + (size_t)h * D;
+      const uint16_t* kn = static_cast<const uint16_t*>(p.knew) + src;
+      const uint16_t* vn = static_cast<const uint16_t*>(p.vnew) + src;
+      adst = p.wplan[b * p.C + j0 + min(al, nj - 1)];
+#pragma unroll
+      for (int i = 0; i < kKI; ++i)
+        akq[i] = *reinterpret_cast<const u32x4_t*>(kn + min(i * kTP + al / kVec, nj - 1) * tstride + 8 * (al % kVec));
+#pragma unroll
+      for (int i = 0; i < kVI; ++i)
+        avq[i] = *reinterpret_cast<const uint32_t*>(vn + min(i * kTV + al / (D / 2), nj - 1) * tstride + 2 * (al % (D / 2)));
+    };
+    auto append_store = [&](int j0) {
+      const int al = opaque_lane(), nj = min(kTok, cb - j0);
+      uint16_t* kp = static_cast<uint16_t*>(const_cast<void*>(p.kpool));
+      uint16_t* vp = static_cast<uint16_t*>(const_cast<void*>(p.vpool));
+#pragma unroll
+      for (int i = 0; i < kKI; ++i) {
+        const int t = i * kTP + al / kVec;
+        const int dest = __shfl(adst, min(t, nj - 1), 64);
+        if (t < nj && dest >= 0)
+          *reinterpret_cast<u32x4_t*>(kp + (slot_index(p, dest >> 4, h) * BS + (dest & 15)) * D + 8 * (al % kVec)) = akq[i];
+      }
+#pragma unroll
+      for (int i = 0; i < kVI; ++i) {
+        const int t = i * kTV + al / (D / 2);
+        const int dest = __shfl(adst, min(t, nj - 1), 64);
+        if (t < nj && dest >= 0) {
+          uint16_t* at = vp + (slot_index(p, dest >> 4, h) * D + 2 * (al % (D / 2))) * BS + (dest & 15);
+          at[0] = (uint16_t)avq[i];
+          at[BS] = (uint16_t)(avq[i] >> 16);
+        }
+      }
+    };
+    auto chunk_page = [&](int pg) {  // the wave's next page of the chunk, from pg on
+      cpg = pg;
+      ca = max(0, pg * BS - start);
+      cb = min(p.C, pg * BS + BS - start);
+      return pg <= (L - 1) >> 4 && (pg < lp1 || lp1 == min((L + BS - 1) / BS, p.max_pages));
+    };
+    auto append_begin = [&]() {
+      static_assert(!kAppend || (PL && !kFp8 && !kF32), "planned kernels over 16-bit pages");
+      if constexpr (kAppend) {
+        int pg = max(start >> 4, lp0);
+        pg += (w - (pg - lp0)) & (NWV - 1);  // pages of the piece go round the waves
+        own = chunk_page(pg);
+        if (kLate && own) append_load(ca);
+        pre = first && !(own && cpg == lp0 + w);
+      }
+    };
+    auto append_end = [&]() {
+      if constexpr (kAppend) {
+        if (!own) return;
+        if (!kLate) append_load(ca);
+        append_store(ca);
+        for (;;) {  // more than kTok tokens in the page, or a chunk of over NWV pages
+          for (int j0 = ca + kTok; j0 < cb; j0 += kTok) {
+            append_load(j0);
+            append_store(j0);
+          }
+          if (!chunk_page(cpg + NWV)) break;
+          append_load(ca);
+          append_store(ca);
+        }
+        // later loads of these pages stay after the stores
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        asm volatile("" ::: "memory");
+      }
+    };
+
     // With four query tiles the row index and the ratio are opaque here, so
     // that what derives from them (the rows 16 nt + i16, the divisor's
     // reciprocal) is recomputed per piece rather than held across the walk.
@@ -964,8 +1075,10 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void attn_mfma_kernel(AttnParams p
           qv[k] = *reinterpret_cast<const uint4*>(qbase + (((size_t)b * p.C + j) * p.Hq + hq) * D + kQV * c);
         }
       }
+      append_begin();
       // Issued after the staging loads, so their wait does not include it.
-      if (first) load_page_phys(buf[0], first_id);
+      if (pre) load_page_phys(buf[0], first_id);
+      append_end();
       __syncthreads();
       if (stid < ntab) sTab[stid] = safe_block(p, tabv, b);
       if (lenv < L) flag_bad_read(p, b);
@@ -977,7 +1090,9 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void attn_mfma_kernel(AttnParams p
       }
     } else {
       const int lenv = !PL && threadIdx.x == 0 && p.lens ? p.lens[sid] : 0x7fffffff;
-      if (first) load_page_phys(buf[0], first_id);
+      append_begin();
+      if (pre) load_page_phys(buf[0], first_id);
+      append_end();
       __syncthreads();
       for (int t = threadIdx.x; t < min(kTabChunk, lp1 - lp0); t += blockDim.x)
         sTab[t] = safe_block(p, table[lp0 + t], b);
@@ -1339,7 +1454,7 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void attn_mfma_kernel(AttnParams p
       // every path, so each page waits only for its own loads (vmcnt(N)), not
       // for the pages prefetched after it (vmcnt(0)).
       // (a planned call's first window: its first page is already in flight)
-      if (!(first && tab0 == lp0)) {
+      if (!(pre && tab0 == lp0)) {
 #pragma unroll
         for (int u = 0; u < kRing - 1; ++u) load_slot(buf[u], u);
       } else {
@@ -1728,16 +1843,16 @@ int launch_valu_q(const AttnParams& p, int kv_dtype, dim3 grid, hipStream_t s, b
   return SPV_OK;
 }
 
-template <int D, bool BAL, int KT, bool PL>
+template <int D, bool BAL, int KT, bool PL, bool AP = false>
 void launch_mfma_mode(const AttnParams& p, int nt, hipStream_t s, dim3 grid, size_t smem) {
   const dim3 blk(kMfmaThreads);
   constexpr int QT = KT == SPV_F16 ? SPV_F16 : SPV_BF16;
   switch (nt) {
-    case 1: launch_attn(attn_mfma_kernel<1, D, QT, BAL, KT, PL>, grid, blk, smem, s, true, true, p); break;
-    case 2: launch_attn(attn_mfma_kernel<2, D, QT, BAL, KT, PL>, grid, blk, smem, s, true, true, p); break;
-    case 3: launch_attn(attn_mfma_kernel<3, D, QT, BAL, KT, PL>, grid, blk, smem, s, true, true, p); break;
+    case 1: launch_attn(attn_mfma_kernel<1, D, QT, BAL, KT, PL, AP>, grid, blk, smem, s, true, true, p); break;
+    case 2: launch_attn(attn_mfma_kernel<2, D, QT, BAL, KT, PL, AP>, grid, blk, smem, s, true, true, p); break;
+    case 3: launch_attn(attn_mfma_kernel<3, D, QT, BAL, KT, PL, AP>, grid, blk, smem, s, true, true, p); break;
     default:  // four query tiles: planned only at head_dim 64 (Plan::plannable)
-      launch_attn(attn_mfma_kernel<4, D, QT, BAL, KT, PL && D != 128>, grid, blk, smem, s, true, true, p);
+      launch_attn(attn_mfma_kernel<4, D, QT, BAL, KT, PL && D != 128, AP && D != 128>, grid, blk, smem, s, true, true, p);
       break;
   }
 }
@@ -1752,6 +1867,13 @@ void launch_mfma(const AttnParams& p, int nt, hipStream_t s) {
   const size_t smem = (size_t)4 * (p.B + 1) * sizeof(int);  // page / piece prefixes, ids, starts
   const int nw = persistent_wgs();
   const bool bal = balanced_split(p, nw);
+  if constexpr (KT != SPV_FP8E4M3) {
+    if (p.plan && p.knew) {
+      if (bal) launch_mfma_mode<D, true, KT, true, true>(p, nt, s, dim3(nw), smem);
+      else launch_mfma_mode<D, false, KT, true, true>(p, nt, s, dim3(nw), smem);
+      return;
+    }
+  }
   if (p.plan) {  // (never with four query tiles at head_dim 128: Plan::plannable)
     if (bal) launch_mfma_mode<D, true, KT, true>(p, nt, s, dim3(nw), smem);
     else launch_mfma_mode<D, false, KT, true>(p, nt, s, dim3(nw), smem);
@@ -1818,7 +1940,8 @@ int spv::verify_attn_impl(void* out, const void* q, int q_dtype, const void* k_p
                      const int32_t* seq_ids, const int32_t* start_pos, const int32_t* seq_lens, int32_t* ctr,
                      int32_t B, int32_t C, int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim,
                      int32_t block_size, int32_t layer, int32_t capacity, int32_t max_ctx, float scale,
-                     const void* plan, void* workspace, size_t workspace_bytes, bool exact_layout, void* stream) {
+                     const void* plan, void* workspace, size_t workspace_bytes, bool exact_layout, void* stream,
+                     const void* k_new, const void* v_new, const int32_t* write_plan) {
   struct Disarm {
     ~Disarm() { g_arm = TimingArm{}; }
   } disarm;  // armed timing events serve this call only, whatever its outcome
@@ -1879,6 +2002,19 @@ int spv::verify_attn_impl(void* out, const void* q, int q_dtype, const void* k_p
   p.scale_log2 = scale * kLog2e;
   // A round's plan serves MFMA calls only (the VALU path has no prologue to skip).
   if (pl.plannable() && plan) p.plan = static_cast<int*>(const_cast<void*>(plan));
+  // A chunk still to be written: by the planned kernels over 16-bit pages
+  // themselves, else in a launch before them.
+  if (k_new) {
+    if (p.plan && (kv_dtype == SPV_BF16 || kv_dtype == SPV_F16) && C <= 64) {
+      p.knew = k_new;
+      p.vnew = v_new;
+      p.wplan = write_plan;
+    } else {
+      const int rc = spv_kv_write_planned(const_cast<void*>(k_pool), const_cast<void*>(v_pool), kv_dtype, k_new, v_new,
+                                          write_plan, B, C, layer, capacity, block_size, num_kv_heads, head_dim, stream);
+      if (rc != SPV_OK) return rc;
+    }
+  }
   if (need > 0) {
     const size_t rows = partial_rows(pl, B, C, num_q_heads, num_kv_heads, nw_layout);
     char* ws = static_cast<char*>(workspace);
@@ -1999,6 +2135,21 @@ int spv_verify_attn_planned(void* out, const void* q, int q_dtype, const void* k
   return spv::verify_attn_impl(out, q, q_dtype, k_pool, v_pool, kv_dtype, kv_scales, block_tables, max_blocks_per_seq,
                           seq_ids, start_pos, seq_lens, ctr, B, C, num_q_heads, num_kv_heads, head_dim, block_size,
                           layer, capacity, max_ctx, scale, plan, workspace, workspace_bytes, false, stream);
+}
+
+int spv_verify_attn_append_planned(void* out, const void* q, int q_dtype, void* k_pool, void* v_pool, int kv_dtype,
+                                   const int32_t* block_tables, int32_t max_blocks_per_seq, const int32_t* seq_ids,
+                                   const int32_t* start_pos, const int32_t* seq_lens, int32_t* ctr, int32_t B,
+                                   int32_t C, int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim,
+                                   int32_t block_size, int32_t layer, int32_t capacity, int32_t max_ctx, float scale,
+                                   const void* plan, const void* k_new, const void* v_new, const int32_t* write_plan,
+                                   void* workspace, size_t workspace_bytes, void* stream) {
+  if (!plan || !k_new || !v_new || !write_plan || kv_dtype == SPV_FP8E4M3) return SPV_ERR_ARG;
+  if (capacity < 1 || block_size < 1 || (long long)capacity * block_size > 0x7fffffffLL) return SPV_ERR_ARG;
+  return spv::verify_attn_impl(out, q, q_dtype, k_pool, v_pool, kv_dtype, nullptr, block_tables, max_blocks_per_seq,
+                          seq_ids, start_pos, seq_lens, ctr, B, C, num_q_heads, num_kv_heads, head_dim, block_size,
+                          layer, capacity, max_ctx, scale, plan, workspace, workspace_bytes, false, stream, k_new,
+                          v_new, write_plan);
 }
 
 }  // extern "C"

@@ -65,6 +65,8 @@ SIGNATURES = {
     "spv_verify_attn_plan_bytes": (S, [I]),
     "spv_verify_attn_plan": (I, [P, I, P, P, P, P, I, I, I, I, I, I, I, I, I, P, S, P]),
     "spv_verify_attn_planned": (I, [P, P, I, P, P, I, P, P, I, P, P, P, P, I, I, I, I, I, I, I, I, I, F, P, P, S, P]),
+    "spv_verify_attn_append_planned": (I, [P, P, I, P, P, I, P, I, P, P, P, P, I, I, I, I, I, I, I, I, I, F, P, P, P, P,
+                                           P, S, P]),
     "spv_prefill_attn": (I, [P, P, P, P, I, P, I, I, I, I, I, F, P]),
     "spv_time_next_attention": (I, [P, P]),
     "spv_verify_attn_static_max_bytes": (S, []),

@@ -33,7 +33,7 @@ import torch
 
 from . import _hip
 from ._hip import call, ptr
-from .kv import PagedKVCache
+from .kv import PagedKVCache, WritePlan
 
 _workspace = _hip.Workspace()
 
@@ -116,6 +116,39 @@ def verify_attention(query_3d: torch.Tensor, kv: PagedKVCache, layer: int,
     ``max_ctx`` must bound ``start + chunk`` for every row. ``plan``: the
     round's ``VerifyPlan`` (same sequences, starts, chunk, heads, max_ctx).
     """
+    return _attend(query_3d, kv, layer, seq_ids, start_positions, max_ctx, scale, out, plan, None)
+
+
+def append_verify_attention(query_3d: torch.Tensor, k_new: torch.Tensor, v_new: torch.Tensor, kv: PagedKVCache,
+                            layer: int, seq_ids: torch.Tensor, start_positions: torch.Tensor, max_ctx: int,
+                            plan: VerifyPlan, write_plan: WritePlan, out: Optional[torch.Tensor] = None
+                            ) -> torch.Tensor:
+    """``kv.write_block_device(layer, seq_ids, start_positions, k_new, v_new,
+    alloc=False, plan=write_plan)``, then ``verify_attention(..., plan=plan)`` of
+    the same chunk: a later layer of a round (engine/model.py:182-190). One
+    launch where both plans serve the call and the planned kernels take its
+    shape (``spv_verify_attn_append_planned``); the two calls otherwise."""
+    B, chunk, hq, d = query_3d.shape
+    shape = (B, chunk, kv.num_kv_heads, d)
+    # ``out`` must not overlap the new keys / values: some workgroups write it
+    # while others still read them.
+    if (B and plan.buf is not None and write_plan.ready and not kv.fp8 and d == kv.head_dim
+            and kv._plannable(chunk) and query_3d.device == kv.device
+            and tuple(k_new.shape) == shape and tuple(v_new.shape) == shape
+            and k_new.device == kv.device and v_new.device == kv.device
+            and (out is None or not {k_new.untyped_storage().data_ptr(), v_new.untyped_storage().data_ptr()}
+                 & {out.untyped_storage().data_ptr()})):
+        write_plan._check(kv.allocator.epoch, B, chunk, seq_ids, start_positions)
+        k_new, v_new = kv._new_kv(k_new, v_new)
+        return _attend(query_3d, kv, layer, seq_ids, start_positions, max_ctx, None, out, plan,
+                       (k_new, v_new, write_plan.rows))
+    kv.write_block_device(layer, seq_ids, start_positions, k_new, v_new, alloc=False, plan=write_plan)
+    return verify_attention(query_3d, kv, layer, seq_ids, start_positions, max_ctx, out=out, plan=plan)
+
+
+def _attend(query_3d, kv, layer, seq_ids, start_positions, max_ctx, scale, out, plan, append) -> torch.Tensor:
+    """``verify_attention``; ``append``: (k_new, v_new, write-plan rows) of a planned
+    call whose chunk is still to be written."""
     B, chunk, hq, d = query_3d.shape
     if d != kv.head_dim or hq % kv.num_kv_heads:
         raise ValueError("query heads/dim do not match the cache")
@@ -145,6 +178,16 @@ def verify_attention(query_3d: torch.Tensor, kv: PagedKVCache, layer: int,
                                                               kv.block_size, int(max_ctx))
     stream = _hip.stream_of(kv.device)
     ws = _workspace.get(ws_bytes, kv.device, stream) if ws_bytes else None
+    if append is not None:
+        kn, vn, rows = append
+        call("spv_verify_attn_append_planned", ptr(out), ptr(q), _hip.dtype_code(q.dtype), ptr(kv.k_pool),
+             ptr(kv.v_pool), kv._dt, ptr(kv.tables_dev), kv.max_blocks_per_seq, ptr(sid_t), ptr(start_t),
+             ptr(kv.lens_dev), ptr(kv.allocator.ctr), B, chunk, hq, kv.num_kv_heads, d, kv.block_size, int(layer),
+             kv.allocator.capacity, int(max_ctx), scale, ptr(plan.buf), ptr(kn), ptr(vn), ptr(rows), ptr(ws),
+             int(ws_bytes), stream)
+        kv._stale = True
+        kv.allocator._stale = True
+        return out
     args = (ptr(out), ptr(q), _hip.dtype_code(q.dtype), ptr(kv.k_pool), ptr(kv.v_pool),
             kv._dt, ptr(kv.scales), ptr(kv.tables_dev), kv.max_blocks_per_seq, ptr(sid_t), ptr(start_t),
             ptr(kv.lens_dev), ptr(kv.allocator.ctr), B, chunk,

@@ -373,12 +373,7 @@ class PagedKVCache:
                 self.allocator._stale = True
                 return
             if plan.ready:
-                if (B, chunk) != (plan.B, plan.C):
-                    raise ValueError("the chunk ({}, {}) does not match its write plan ({}, {})".format(
-                        B, chunk, plan.B, plan.C))
-                if plan.epoch != self.allocator.epoch or plan.key != WritePlan._key(seq_ids, start_positions):
-                    raise ValueError("the write plan was recorded for another chunk, or before a later "
-                                     "call that may have freed its blocks")
+                plan._check(self.allocator.epoch, B, chunk, seq_ids, start_positions)
                 call("spv_kv_write_planned", ptr(self.k_pool), ptr(self.v_pool), self._dt, ptr(k_new), ptr(v_new),
                      ptr(plan.rows), B, chunk, int(layer), self.allocator.capacity, self.block_size,
                      self.num_kv_heads, self.head_dim, self._stream())
@@ -714,6 +709,14 @@ class WritePlan:
             self.rows = torch.empty(max(B * C, 64), dtype=torch.int32, device=device)
         self.B, self.C = B, C
         self.ready = False
+
+    def _check(self, epoch: int, B: int, chunk: int, seq_ids: torch.Tensor, starts: torch.Tensor) -> None:
+        if (B, chunk) != (self.B, self.C):
+            raise ValueError("the chunk ({}, {}) does not match its write plan ({}, {})".format(
+                B, chunk, self.B, self.C))
+        if self.epoch != epoch or self.key != WritePlan._key(seq_ids, starts):
+            raise ValueError("the write plan was recorded for another chunk, or before a later "
+                             "call that may have freed its blocks")
 
     def _record(self, epoch: int, seq_ids: torch.Tensor, starts: torch.Tensor) -> None:
         self.epoch = epoch

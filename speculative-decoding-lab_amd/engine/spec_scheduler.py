@@ -37,7 +37,7 @@ import torch
 
 from . import _hip
 from ._hip import call, ptr
-from .attention import VerifyPlan, verify_attention
+from .attention import VerifyPlan, append_verify_attention, verify_attention
 from .kv import PagedKVCache, WritePlan
 
 _workspace = _hip.Workspace()
@@ -353,6 +353,13 @@ class VerifyStep:
             mark()
             kl = k_layers[layer].to(self.kv.dtype).contiguous()
             vl = v_layers[layer].to(self.kv.dtype).contiguous()
+            o = None if outs is None else outs[layer]
+            if plan is not None and events is None:
+                # a later layer: its append and attention in one launch (timed
+                # rounds keep them apart, with an event between)
+                results.append(append_verify_attention(q_layers[layer], kl, vl, self.kv, layer, sid_t, st_t, max_ctx,
+                                                       plan, self._write_plan, out=o))
+                continue
             if layer == 0 and pending is not None:
                 # the previous round's commit, then this round's allocating append: one launch
                 self.kv.rewind_append_device(sid_t, pending.new_len, pending.finished, st_t, kl, vl,
@@ -365,7 +372,7 @@ class VerifyStep:
                 plan = VerifyPlan(self.kv, sid_t, st_t, chunk, int(q_layers[layer].shape[2]), max_ctx)
             mark()
             results.append(verify_attention(q_layers[layer], self.kv, layer, sid_t, st_t, max_ctx,
-                                            out=None if outs is None else outs[layer], plan=plan))
+                                            out=o, plan=plan))
         mark()
         return results
 
@@ -505,11 +512,16 @@ class DraftLoop:
             outs_s = []
             plan = None
             for layer in range(len(q_steps[s])):
+                o = None if attn_out is None else attn_out[s][layer]
+                if plan is not None:  # a later layer: its append and attention in one launch
+                    outs_s.append(append_verify_attention(q_steps[s][layer], k_steps[s][layer], v_steps[s][layer], kv,
+                                                          layer, seq_ids, pos, max_ctx + s + 1, plan, self._write_plan,
+                                                          out=o))
+                    continue
                 kv.write_block_device(layer, seq_ids, pos, k_steps[s][layer], v_steps[s][layer], alloc=layer == 0,
                                       plan=self._write_plan)
                 if plan is None:  # the step's attention plan, once its blocks exist
                     plan = VerifyPlan(kv, seq_ids, pos, 1, int(q_steps[s][layer].shape[2]), max_ctx + s + 1)
-                o = None if attn_out is None else attn_out[s][layer]
                 outs_s.append(verify_attention(q_steps[s][layer], kv, layer, seq_ids, pos, max_ctx + s + 1, out=o,
                                                plan=plan))
             outs.append(outs_s)
