@@ -57,6 +57,12 @@ const char* spv_version(void);
 
 /* ------------------------------------------------------------------ pool */
 
+/* out[0 .. n) = host[0 .. n) in stream order, n <= SPV_PUT_INTS_MAX: the values
+ * travel in the launch's arguments, so `host` may be changed on return and the
+ * call never waits. */
+#define SPV_PUT_INTS_MAX 960
+int spv_put_ints(int32_t* out, const int32_t* host, int32_t n, void* stream);
+
 /* BlockAllocator.__init__ free list [0..cap-1] (engine/kv.py:48-55) and
  * PagedKVCache.reset of the free list (engine/kv.py:173-183). */
 int spv_pool_init(int32_t* free_stack, int32_t* free_flag, int32_t* ctr,

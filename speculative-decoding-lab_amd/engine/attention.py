@@ -79,8 +79,7 @@ class VerifyPlan:
                  start_positions: Union[Sequence[int], torch.Tensor], chunk: int, num_q_heads: int,
                  max_ctx: int, buf: Optional[torch.Tensor] = None) -> None:
         self.kv = kv
-        self.seq_ids = _hip.i32(seq_ids, kv.device)
-        self.start = _hip.i32(start_positions, kv.device)
+        self.seq_ids, self.start = _hip.i32s(kv.device, seq_ids, start_positions)
         self.B = int(self.seq_ids.numel())
         self.chunk, self.num_q_heads, self.max_ctx = int(chunk), int(num_q_heads), int(max_ctx)
         self.ws_bytes: Optional[int] = None  # the calls' workspace size, asked by the first
@@ -163,8 +162,7 @@ def _attend(query_3d, kv, layer, seq_ids, start_positions, max_ctx, scale, out, 
         plan.check(kv, B, chunk, hq, int(max_ctx))
         sid_t, start_t = plan.seq_ids, plan.start
     else:
-        sid_t = _hip.i32(seq_ids, kv.device)
-        start_t = _hip.i32(start_positions, kv.device)
+        sid_t, start_t = _hip.i32s(kv.device, seq_ids, start_positions)
     if max_ctx > kv.max_blocks_per_seq * kv.block_size:
         kv._grow_width(-(-max_ctx // kv.block_size))
     scale = 1.0 / math.sqrt(d) if scale is None else float(scale)

@@ -313,8 +313,7 @@ class SpecContinuousDriver:
         if gpu_timing == "round":  # the round's span only: no event between its kernels
             round_evs = [torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)]
             round_evs[0].record()
-        sid_t = _hip.i32(sids, dev)
-        st_t = _hip.i32(starts, dev)
+        sid_t, st_t = _hip.i32s(dev, sids, starts)
         d_outs = cu = d_stats = d_flags = None
         if self.draft_kv is not None:
             # gamma draft steps from the draft cache's length (== start); the

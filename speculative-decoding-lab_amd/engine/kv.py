@@ -195,12 +195,12 @@ class PagedKVCache:
     def _refresh(self) -> None:
         if self._stale:
             n = len(self._nb)
-            self._nb = self.nblocks_dev[:n].tolist()
-            self._lens = self.lens_dev[:n].tolist()
-            self.allocator._stale = True
-            self.allocator._refresh()
+            # one read for the lengths, the counters and the free count
+            got = torch.cat((self.nblocks_dev[:n], self.lens_dev[:n], self.allocator.ctr)).tolist()
+            self._nb, self._lens, ctr = got[:n], got[n:2 * n], got[2 * n:]
+            self.allocator._free_count = ctr[_hip.CTR_TOP]
+            self.allocator._stale = False
             self._stale = False
-            ctr = self.allocator.ctr.tolist()
             words = (_hip.CTR_EXHAUSTED, _hip.CTR_OVERFLOW, _hip.CTR_BAD_READ, _hip.CTR_ALIGN)
             if not any(ctr[w] for w in words):
                 return
@@ -321,8 +321,7 @@ class PagedKVCache:
             if k_new.device != self.device or v_new.device != self.device:
                 raise ValueError("k/v must live on {}".format(self.device))
             k_new, v_new = self._new_kv(k_new, v_new)
-        sid_t = _hip.i32(seq_ids, self.device)
-        start_t = _hip.i32(starts, self.device)
+        sid_t, start_t = _hip.i32s(self.device, seq_ids, starts)
         self._launch_append(layer, sid_t, start_t, k_new, v_new, B, chunk, 1 if sum(grants) else 0, fail)
         # Mirrors: allocation, then the lengths the (possibly truncated) writes reach.
         for b, sid in enumerate(seq_ids):
@@ -446,9 +445,7 @@ class PagedKVCache:
             return
         nl = [-1] * n if new_lens is None else [int(x) for x in new_lens]
         fin = [0] * n if finished is None else [1 if f else 0 for f in finished]
-        sid_t = _hip.i32(seq_ids, self.device)
-        nl_t = _hip.i32(nl, self.device)
-        fin_t = _hip.i32(fin, self.device)
+        sid_t, nl_t, fin_t = _hip.i32s(self.device, seq_ids, nl, fin)
         self.allocator.epoch += 1
         call("spv_kv_rewind", ptr(self.tables_dev), self._maxb, ptr(self.nblocks_dev),
              ptr(self.lens_dev), ptr(self.allocator.free_stack), ptr(self.allocator.free_flag),

@@ -330,8 +330,7 @@ class VerifyStep:
         (``2 * layers + 1`` events)."""
         chunk = self.gamma + 1
         max_ctx = max(int(s) for s in start_positions) + chunk
-        sid_t = _hip.i32(seq_ids, self.kv.device)
-        st_t = _hip.i32(start_positions, self.kv.device)
+        sid_t, st_t = _hip.i32s(self.kv.device, seq_ids, start_positions)
         results = []
         self.kv._grow_width(-(-max_ctx // self.kv.block_size))
 
@@ -387,8 +386,7 @@ class VerifyStep:
         (``verify_sample``)."""
         self.flush()
         dev = self.kv.device
-        sid_t = _hip.i32(seq_ids, dev)
-        st_t = _hip.i32(start_positions, dev)
+        sid_t, st_t = _hip.i32s(dev, seq_ids, start_positions)
         rem_t = None if remaining is None else _hip.i32(remaining, dev)
         res = verify_sample(target_logits, draft_logits, proposals, u, noise, self.temperature,
                             start_pos=st_t, remaining=rem_t, eos_id=self.eos_id, validate=False,
