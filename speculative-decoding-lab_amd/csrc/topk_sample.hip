@@ -5,8 +5,8 @@
 // With top-k on, at most a few hundred values of a 151,936-entry row survive,
 // so the filtered rows are never written: one launch reads every row once and
 // keeps its survivors.
-//   1. A workgroup per row piece holds the piece in registers (up to 160 values
-//      per thread, all loads in flight). The k-th largest of 1,024 group maxima
+//   1. A workgroup per row piece holds the piece in registers (64 values per
+//      thread for most calls, all loads in flight). The k-th largest of 1,024 group maxima
 //      bounds the piece's k-th largest value from below, so every value at or
 //      above it (a few more than k) is a candidate and the rest cannot survive.
 //   2. The last piece of a row takes the candidates of all pieces, selects the
@@ -17,8 +17,13 @@
 //      torch's arithmetic (every other token's key is exactly 0) and commits.
 // The rows are read once and nothing else of their size moves: the launch is
 // bound by HBM. B = 32, gamma = 5, V = 151,936, T = 0.8, top_k 50, top_p 0.9
-// (233 MB): 97 us per call against 662 for filtering all rows into memory
+// (233 MB): 75 us per call against 662 for filtering all rows into memory
 // (five passes a row), their statistics and the race, 900 when a draw was re-raced.
+// Of the 75 the reading takes 38; the rest is the tail of the last rows -- bound,
+// publication, row, sequence, each a chain of barriers and uncached round trips
+// -- and three empty launches of the general kernels. With searches that halved
+// the key space (14 and 19 barriers) and a row's lists read one dependent load
+// at a time the call took 98.
 //
 // Whatever the short form does not cover -- a NaN or infinite logit, more ties
 // or candidates than the lists hold, a row with nothing finite, a race noise
@@ -37,18 +42,23 @@ constexpr int kTThreads = 256;
 constexpr int kTWaves = kTThreads / 64;
 // Largest top_k of the short form (and the temperatures it takes: those whose
 // quotients stay far from overflow and underflow). B = 32, gamma = 5,
-// V = 151,936, T = 0.8, top_p 0.9, us per call: top_k 20 95, 50 98, 200 120,
-// 400 176, 512 200 (the lists grow with it), against 628 for the general path;
-// B = 1: 35 to 68 against 256.
+// V = 151,936, T = 0.8, top_p 0.9, us per call: top_k 20 72, 50 76, 200 106,
+// 400 153, 512 193 (the lists grow with it), against 605 for the general path;
+// B = 1: 33 to 67 against 256.
 constexpr int kTopkMax = 512;
 constexpr float kTempMin = 0x1p-10f, kTempMax = 0x1p10f;
 constexpr int kPieceCap = 1024;  // candidates of a piece
 constexpr int kRowCap = 4096;    // candidates of a row
+constexpr int kRowCapMid = 2048; // the same where kVecMid pieces are held
 constexpr int kKeepCap = 1024;   // kept values of a row
 constexpr int kMaxPieces = 16;
-// float4 per thread of a piece: 40 (40,960 values) when the batch's rows fill
-// the CUs, 10 for a few rows.
-constexpr int kVecBig = 40, kVecSmall = 10;
+// float4 per thread of a piece: 16 (16,384 values) when the batch's rows fill
+// the CUs, 10 for a few rows, and 40 where the lists of 16 would not hold a
+// large top_k's candidates. 16 take 128 registers, so four workgroups of a CU
+// overlap one's loads with the others' selection (B = 32, top_k 50, us per call:
+// 77 with 16, 79 with 20, 87 with 40 and two workgroups per CU).
+constexpr int kVecBig = 40, kVecMid = 16, kVecSmall = 10;
+constexpr int row_cap(int nvec) { return nvec == kVecMid ? kRowCapMid : kRowCap; }
 constexpr size_t kMaxListBytes = (size_t)256 << 20;
 constexpr int kMaxRows = 65536;  // row counters
 
@@ -85,36 +95,106 @@ __device__ __forceinline__ int entry_idx(unsigned long long e) { return (int)(0x
 // The first key above -inf's.
 constexpr uint32_t kFirstKey = 0x00800000u;
 
+// A bracket of the want-th largest of the workgroup's keys: at least `want`
+// (c of them) are >= lo, fewer are >= hi; lo = 0 when fewer than `want` are
+// finite. One histogram of the keys over 256 equal bins of their range and its
+// suffix sums, three barriers: halving the key space took 14 (a piece's bound) to
+// 19 (a row's threshold) of them, about 0.4 us each.
+struct Bracket {
+  uint32_t lo, hi;
+  int c;
+};
+struct BracketLds {
+  int hist[256];
+  uint32_t lo[kTWaves], hi[kTWaves];
+};
+template <int N>
+__device__ __forceinline__ Bracket block_bracket(const uint32_t (&key)[N], int want, BracketLds& s) {
+  const int t = threadIdx.x, lane = t & 63;
+  uint32_t kmin = 0xffffffffu, kmax = 0;
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+    if (key[i] >= kFirstKey) {
+      kmin = min(kmin, key[i]);
+      kmax = max(kmax, key[i]);
+    }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    kmin = min(kmin, (uint32_t)__shfl_xor((int)kmin, o, 64));
+    kmax = max(kmax, (uint32_t)__shfl_xor((int)kmax, o, 64));
+  }
+  s.hist[t] = 0;
+  if (lane == 0) {
+    s.lo[t >> 6] = kmin;
+    s.hi[t >> 6] = kmax;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < kTWaves; ++w) {
+    kmin = min(kmin, s.lo[w]);
+    kmax = max(kmax, s.hi[w]);
+  }
+  // bins of 2^sh keys: the range's top 8 bits
+  const int sh = kmax > kmin ? max(0, 24 - __clz((int)(kmax - kmin))) : 0;
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+    if (key[i] >= kFirstKey) atomicAdd(&s.hist[(key[i] - kmin) >> sh], 1);
+  __syncthreads();
+  // lane l: bins 255 - 4 l down to 252 - 4 l, the largest keys in lane 0
+  int n[4], sum = 0;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    n[j] = s.hist[255 - 4 * lane - j];
+    sum += n[j];
+  }
+  int incl = sum;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int y = __shfl_up(incl, o, 64);
+    if (lane >= o) incl += y;
+  }
+  const unsigned long long enough = __ballot(incl >= want);
+  __syncthreads();  // the buffers are free again
+  if (!enough) return Bracket{0u, kFirstKey, 0};
+  int c = incl - sum, bin = 255 - 4 * lane;
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    if (c < want) {
+      c += n[j];
+      bin = 255 - 4 * lane - j;
+    }
+  const int from = __ffsll(enough) - 1;
+  c = __shfl(c, from, 64);
+  bin = __shfl(bin, from, 64);
+  const unsigned long long hi = (unsigned long long)kmin + ((unsigned long long)(bin + 1) << sh);
+  return Bracket{kmin + ((uint32_t)bin << sh), hi > 0xffffffffull ? 0xffffffffu : (uint32_t)hi, c};
+}
+
 // A bound t such that at least `want` and at most about `most` of the
 // workgroup's keys are >= t (exactly the want-th largest key when most ==
-// want, unless ties make more), or 0 when fewer than `want` are finite: a
-// bisection over the key space, one count of the workgroup per step.
+// want, unless ties make more), or 0 when fewer than `want` are finite: the
+// bracket, halved (a count of the workgroup per step) while it holds more.
 template <int N>
-__device__ __forceinline__ uint32_t block_bound(const uint32_t (&key)[N], int want, int most, int (*s_cnt)[kTWaves]) {
+__device__ __forceinline__ uint32_t block_bound(const uint32_t (&key)[N], int want, int most, BracketLds& s_br,
+                                                int (*s_cnt)[kTWaves]) {
+  Bracket br = block_bracket<N>(key, want, s_br);
   int par = 0;
-  auto count = [&](uint32_t t) {
+  while (br.c > most && br.hi - br.lo > 1) {
+    const uint32_t mid = br.lo + (br.hi - br.lo) / 2;
     int c = 0;
 #pragma unroll
-    for (int i = 0; i < N; ++i) c += __popcll(__ballot(key[i] >= t));
+    for (int i = 0; i < N; ++i) c += __popcll(__ballot(key[i] >= mid));
     if ((threadIdx.x & 63) == 0) s_cnt[par][threadIdx.x >> 6] = c;
     __syncthreads();
     int n = 0;
 #pragma unroll
     for (int w = 0; w < kTWaves; ++w) n += s_cnt[par][w];
     par ^= 1;  // the next count writes the other buffer: one barrier per step
-    return n;
-  };
-  uint32_t lo = kFirstKey, hi = 0xffffffffu;
-  int c = count(lo);
-  if (c < want) lo = 0, c = 0;
-  while (c > most && hi - lo > 1) {
-    const uint32_t mid = lo + (hi - lo) / 2;
-    const int cm = count(mid);
-    if (cm >= want) lo = mid, c = cm;
-    else hi = mid;
+    if (n >= want) br.lo = mid, br.c = n;
+    else br.hi = mid;
   }
   __syncthreads();  // the buffers are free again
-  return lo;
+  return br.lo;
 }
 
 // The decision, the race over the raced row's kept list and the commit of one
@@ -263,16 +343,17 @@ __device__ __forceinline__ int block_sum(int v, int (*s_cnt)[kTWaves]) {
 // grid: per sequence (2 gamma + 1) rows and the noise row, `pieces` workgroups
 // each; sequences one after another.
 template <int NVEC, bool VEC, bool UNIT>
-__global__ __launch_bounds__(kTThreads, 2) void topk_sample_kernel(TkArgs a) {
-  constexpr int kGroups = NVEC == kVecBig ? 4 : 5, kPer = NVEC / kGroups;  // group maxima per thread
+__global__ __launch_bounds__(kTThreads, NVEC == kVecMid ? 4 : 2) void topk_sample_kernel(TkArgs a) {
+  constexpr int kCap = row_cap(NVEC);
+  constexpr int kGroups = NVEC != kVecSmall ? 4 : 5, kPer = NVEC / kGroups;  // group maxima per thread
   static_assert(NVEC % kGroups == 0 && kGroups * kTThreads >= 2 * kTopkMax, "enough group maxima for any top_k");
   const int gamma = a.d.gamma, C = gamma + 1, nr = 2 * gamma + 1, V = a.d.V, P = a.pieces, t = threadIdx.x;
   const int b = blockIdx.x / ((nr + 1) * P), rem = blockIdx.x - b * (nr + 1) * P, r = rem / P, pc = rem - r * P;
-  __shared__ unsigned long long s_row[kRowCap];  // the piece's candidates, then the row's
+  __shared__ unsigned long long s_row[kCap];  // the piece's candidates, then the row's
   __shared__ unsigned long long s_keep[kKeepCap];
   __shared__ int s_cnt[2][kTWaves];
+  __shared__ BracketLds s_br;
   __shared__ double s_scan[kTWaves];
-  __shared__ int s_pn[kMaxPieces];
   __shared__ float s_zx;
   __shared__ int s_n, s_last;
   const float* src = r < C ? a.d.target + ((size_t)b * C + r) * V
@@ -335,7 +416,7 @@ __global__ __launch_bounds__(kTThreads, 2) void topk_sample_kernel(TkArgs a) {
       gk[g] = order_key(m);
     }
     if (t == 0) s_n = 0;
-    const uint32_t bound = block_bound<kGroups>(gk, a.top_k, a.top_k + a.top_k / 16 + 16, s_cnt);
+    const uint32_t bound = block_bound<kGroups>(gk, a.top_k, a.top_k + a.top_k / 16 + 16, s_br, s_cnt);
     // On the raw logits: lowered so that no logit whose quotient by T rounds to
     // the bound's is left out (2 ulp of the quotient; the constant covers
     // quotients that underflow).
@@ -364,8 +445,16 @@ __global__ __launch_bounds__(kTThreads, 2) void topk_sample_kernel(TkArgs a) {
     if (t == 0) store_coherent_b64(rc, (crow + pc) * sizeof(int2), u32x2_t{(unsigned)(nc <= kPieceCap ? nc : -1), 0u});
     if (!arrive_last(a.cnt_row + (size_t)b * nr + r, P, &s_last)) return;
 
-    // 2. the row: every piece's candidates, scaled
-    if (t < P) s_pn[t] = (int)load_coherent_b64(rc, (crow + t) * sizeof(int2)).x;
+    // 2. the row: every piece's candidates, scaled. 256 / P threads take a piece;
+    // its count and their first kAhead entries come in one round trip (what lies
+    // past the count is dropped).
+    constexpr int kAhead = 4;
+    const int tp = kTThreads / P, q = t / tp, sub = t - q * tp;
+    const size_t lpiece = lrow + (size_t)min(q, P - 1) * kPieceCap;
+    int pn = (int)load_coherent_b64(rc, (crow + min(q, P - 1)) * sizeof(int2)).x;
+    u32x2_t ahead[kAhead];
+#pragma unroll
+    for (int e = 0; e < kAhead; ++e) ahead[e] = load_coherent_b64(rl, (lpiece + sub + e * tp) * sizeof(uint2));
     const int j = r < gamma ? r : r >= C ? r - C : -1;  // the row's proposal
     const int xj = j >= 0 ? a.d.proposals[(size_t)b * gamma + j] : -1;
     if (t == 0) {
@@ -373,41 +462,56 @@ __global__ __launch_bounds__(kTThreads, 2) void topk_sample_kernel(TkArgs a) {
       s_zx = -INFINITY;
     }
     __syncthreads();
-    int total = 0;
-    bool bad = false;
-    for (int i = 0; i < P; ++i) {
-      bad |= s_pn[i] < 0;
-      total += s_pn[i];
+    bool odd = false;
+    auto take = [&](const u32x2_t& c) {
+      const float z = __uint_as_float(c.x), x = UNIT ? z : z / a.d.tf;
+      odd |= !(fabsf(x) < INFINITY);  // NaN, or infinite
+      const int at = atomicAdd(&s_n, 1);
+      if (at < kCap) s_row[at] = pack_entry(order_key(x), (int)c.y);
+    };
+    if (q < P) {
+      odd |= pn < 0;
+#pragma unroll
+      for (int e = 0; e < kAhead; ++e)
+        if (sub + e * tp < pn) take(ahead[e]);
+      for (int i = sub + kAhead * tp; i < pn; i += tp) take(load_coherent_b64(rl, (lpiece + i) * sizeof(uint2)));
     }
-    bad |= total < 1 || total > kRowCap;
+    bool bad = __syncthreads_or(odd);
+    const int total = s_n;
+    bad |= total < 1 || total > kCap;
     RowDesc out{};
     if (!bad) {
-      bool odd = false;
-      for (int i = t; i < total; i += kTThreads) {
-        int q = 0, at = i;
-        while (at >= s_pn[q]) at -= s_pn[q++];
-        const u32x2_t c = load_coherent_b64(rl, (lrow + (size_t)q * kPieceCap + at) * sizeof(uint2));
-        const float z = __uint_as_float(c.x), x = UNIT ? z : z / a.d.tf;
-        odd |= !(fabsf(x) < INFINITY);  // NaN, or infinite
-        s_row[i] = pack_entry(order_key(x), (int)c.y);
-      }
-      bad = __syncthreads_or(odd);
-    }
-    if (!bad) {
-      // the k-th largest, then what is at or above it
-      uint32_t thr;
-      if (total <= 4 * kTThreads) {
-        uint32_t key[4];
+      // What is at or above the k-th largest. The entries from the bracket's
+      // lower end on (a few more than k) are sorted, and the k-th of them is
+      // the threshold; where the lists do not hold them the exact bound is
+      // searched first.
+      uint32_t thr = 0;
+      int held;  // entries >= thr
+      auto bracket = [&](auto& key, bool exact) {
+        constexpr int N = sizeof(key) / sizeof(key[0]);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) key[i] = t + i * kTThreads < total ? entry_key(s_row[t + i * kTThreads]) : 0u;
-        thr = block_bound<4>(key, a.top_k, a.top_k, s_cnt);
-      } else {
-        uint32_t key[kRowCap / kTThreads];
-#pragma unroll
-        for (int i = 0; i < kRowCap / kTThreads; ++i)
-          key[i] = t + i * kTThreads < total ? entry_key(s_row[t + i * kTThreads]) : 0u;
-        thr = block_bound<kRowCap / kTThreads>(key, a.top_k, a.top_k, s_cnt);
-      }
+        for (int i = 0; i < N; ++i) key[i] = t + i * kTThreads < total ? entry_key(s_row[t + i * kTThreads]) : 0u;
+        if (exact) {
+          thr = block_bound<N>(key, a.top_k, a.top_k, s_br, s_cnt);
+          return;
+        }
+        const Bracket br = block_bracket<N>(key, a.top_k, s_br);
+        thr = br.lo;
+        held = br.lo ? br.c : total;
+      };
+      auto find = [&](bool exact) {
+        if (total <= 4 * kTThreads) {
+          uint32_t key[4];
+          bracket(key, exact);
+        } else {
+          uint32_t key[kCap / kTThreads];
+          bracket(key, exact);
+        }
+      };
+      find(false);
+      if (held > kKeepCap) find(true);
+      if (t == 0) s_n = 0;
+      __syncthreads();
       for (int i = t; i < total; i += kTThreads) {
         const unsigned long long c = s_row[i];
         if (entry_key(c) >= thr) {
@@ -416,7 +520,7 @@ __global__ __launch_bounds__(kTThreads, 2) void topk_sample_kernel(TkArgs a) {
         }
       }
       __syncthreads();
-      const int nk = s_n;
+      int nk = s_n;
       bad = nk > kKeepCap;
       if (!bad) {
         // sorted by value, equal values by index: every entry's rank
@@ -427,6 +531,12 @@ __global__ __launch_bounds__(kTThreads, 2) void topk_sample_kernel(TkArgs a) {
           s_row[rank] = c;
         }
         __syncthreads();
+        if (thr && nk > a.top_k) {  // cut at the k-th value; its ties stay
+          const uint32_t kth = entry_key(s_row[a.top_k - 1]);
+          int ties = 0;
+          for (int i = a.top_k + t; i < nk; i += kTThreads) ties += entry_key(s_row[i]) == kth;
+          nk = a.top_k + block_sum(ties, s_cnt);
+        }
         const float M = key_value(entry_key(s_row[0]));
         int keep = nk, amb = 0;
         const int per = (nk + kTThreads - 1) / kTThreads, q0 = min(nk, t * per), q1 = min(nk, q0 + per);
@@ -489,14 +599,16 @@ TkPlan tk_plan(int B, int gamma, int V, float temperature, int top_k) {
       !(temperature <= kTempMax))
     return {0, 0};
   // candidates of a row over n pieces, with a third to spare
-  auto fits = [&](int n) {
-    return n <= kMaxPieces && (long long)n * (top_k + top_k / 16 + 16) * 4 / 3 <= kRowCap &&
+  auto fits = [&](int n, int nvec) {
+    return n <= kMaxPieces && (long long)n * (top_k + top_k / 16 + 16) * 4 / 3 <= row_cap(nvec) &&
            rows * n * kPieceCap * sizeof(uint2) <= kMaxListBytes;
   };
   // One float4 less than the registers hold per thread, so that an uneven cut fits.
-  const int small = ceil_of(V, 4 * kTThreads * kVecSmall - 4), big = ceil_of(V, 4 * kTThreads * kVecBig - 4);
-  if (fits(small) && rows * small <= 1024) return {small, kVecSmall};
-  if (fits(big)) return {big, kVecBig};
+  auto pieces = [&](int nvec) { return ceil_of(V, 4 * kTThreads * nvec - 4); };
+  const int small = pieces(kVecSmall), mid = pieces(kVecMid), big = pieces(kVecBig);
+  if (fits(small, kVecSmall) && rows * small <= 1024) return {small, kVecSmall};
+  if (fits(mid, kVecMid)) return {mid, kVecMid};
+  if (fits(big, kVecBig)) return {big, kVecBig};
   return {0, 0};
 }
 
@@ -592,6 +704,7 @@ int spv_verify_sample_filtered(const float* target, const float* draft, float te
     a.desc = reinterpret_cast<RowDesc*>(ws + l.desc);
     const int grid = (rows + B) * pl.pieces;
     if (pl.nvec == kVecBig) launch_tk<kVecBig>(a, grid, (hipStream_t)stream);
+    else if (pl.nvec == kVecMid) launch_tk<kVecMid>(a, grid, (hipStream_t)stream);
     else launch_tk<kVecSmall>(a, grid, (hipStream_t)stream);
     SPV_CHECK_LAUNCH();
   }

@@ -204,6 +204,10 @@ def _general(t, d, x, u, noise, T, top_k, top_p):
     (1, 32, 10236, 1.0, 20, 1.0),        # one full small piece; the longest draft
     (1, 3, 10240, 0.5, 512, 0.8),        # one value more than a piece; the largest top_k
     (40, 5, 40957, 1.0, 100, 0.9),       # two large pieces, unaligned rows
+    (60, 5, 16380, 1.0, 30, 0.9),        # one full middle piece
+    (60, 5, 16381, 0.9, 30, 0.8),        # one value more, unaligned
+    (20, 5, 151936, 1.0, 129, 0.9),      # the largest top_k of the middle pieces, and one more
+    (20, 5, 151936, 1.0, 130, 0.9),
     (64, 5, 151936, 0.8, 50, 0.9),       # the fused workload
     (20, 2, 151936, 1.0, 513, 0.9),      # top_k above the short form's
 ])
