@@ -151,7 +151,11 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_mfma_kernel(PrefillParams
   // 1,303 against 170 / 480 / 1,349 us in slice order). Otherwise: slice
   // order, each slice from its longest block down.
   const int S = p.B * p.Hkv, nblk = p.nblk, id = (int)blockIdx.x;
-  __shared__ int s_equal, s_sl, s_d;
+  // (The wave's sums and maxima go through DPP: as shuffles, 54 to 80 dependent
+  // LDS round trips, this took 2-3 us of every workgroup, one after another on
+  // a CU. Four prompts of 721 to 5,116, 16/2 heads of 128, bf16: 249 -> 242 us; 16
+  // of 32 to 512, 14/2 heads of 64, fp16: 21.0 -> 19.8.)
+  __shared__ int s_equal, s_sl, s_d, s_len;
   if (threadIdx.x < 64) {
     const int i = (int)threadIdx.x;
     int lo = 0x7fffffff, hi = -1;
@@ -160,42 +164,28 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_mfma_kernel(PrefillParams
       lo = min(lo, Lb);
       hi = max(hi, Lb);
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      lo = min(lo, __shfl_xor(lo, o, 64));
-      hi = max(hi, __shfl_xor(hi, o, 64));
+    lo = 0x7fffffff - lane63(wave_incl_max(0x7fffffff - lo));  // lengths are in [0, Lc]
+    hi = lane63(wave_incl_max(max(hi, 0)));
+    if (i == 0) {
+      s_equal = lo == hi;
+      s_len = lo;
     }
-    if (i == 0) s_equal = lo == hi;
-    if (p.B <= 64) {
+    if (p.B <= 64 && !(lo == hi && (S % 8 == 0 || 8 % S == 0))) {
       // Lane i: sequence i's blocks with rows (nb) and its last block's tile
       // count (T). Block j < nb has ceil(min(L, BM (j + 1)) / 64) tiles, so
       // the blocks with at least c <= T tiles are j >= 64 (c - 1) / BM.
       const int BM = p.BM, Hkv = p.Hkv;
       const int Li = i < p.B ? min(max(p.lengths[i], 0), p.Lc) : 0;
       const int nb = (Li + BM - 1) / BM, T = (Li + 63) / 64;
-      auto wsum = [](int x) {
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
-        return x;
-      };
-      auto excl = [&](int x) {  // exclusive prefix sum over the lanes
-        int v = x;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-          const int y = __shfl_up(v, o, 64);
-          if (i >= o) v += y;
-        }
-        return v - x;
-      };
+      auto wsum = [](int x) { return lane63(wave_incl_sum(x)); };
+      auto excl = [](int x) { return wave_incl_sum(x) - x; };  // exclusive prefix sum over the lanes
       auto first = [&](int c) { return 64 * (c - 1) / BM; };
       auto atleast = [&](int c) { return Hkv * wsum(c <= T ? nb - first(c) : 0); };  // items with >= c tiles
       if (i == 0) s_sl = S;  // past every item (the grid is padded to whole rounds of 8)
       const int total = atleast(1);
       if (id < total) {
         // the tile count c of item id: the largest c with more than id items of >= c tiles
-        int c = 1, top = T;
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) top = max(top, __shfl_xor(top, o, 64));
+        int c = 1, top = lane63(wave_incl_max(T));
         while (c < top) {
           const int mid = (c + top + 1) >> 1;
           if (atleast(mid) > id) c = mid;
@@ -208,6 +198,7 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_mfma_kernel(PrefillParams
         if (r >= pre && r < pre + Hkv * n) {
           s_sl = i * Hkv + (r - pre) / n;
           s_d = nblk - 1 - (last - (r - pre) % n);
+          s_len = Li;
         }
       } else {
         const int r = id - total, ne = nblk - nb;  // the blocks without rows
@@ -215,6 +206,7 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_mfma_kernel(PrefillParams
         if (r >= pre && r < pre + Hkv * ne) {
           s_sl = i * Hkv + (r - pre) / ne;
           s_d = nblk - 1 - (nb + (r - pre) % ne);
+          s_len = Li;
         }
       }
     }
@@ -240,7 +232,8 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_mfma_kernel(PrefillParams
   const int b = __builtin_amdgcn_readfirstlane(sl / p.Hkv), hk = __builtin_amdgcn_readfirstlane(sl % p.Hkv);
   const int blk = __builtin_amdgcn_readfirstlane(nblk - 1 - d);
   const int p0 = blk * p.BM;
-  const int L = min(max(p.lengths[b], 0), p.Lc);  // never a key beyond the chunk
+  // the length (never a key beyond the chunk): in hand but for a large ragged batch
+  const int L = s_equal || p.B <= 64 ? __builtin_amdgcn_readfirstlane(s_len) : min(max(p.lengths[b], 0), p.Lc);
   const int ratio = p.ratio, Hq = p.Hq, Hkv = p.Hkv, Lc = p.Lc;
   const uint16_t* qb = static_cast<const uint16_t*>(p.q);
   const uint16_t* kb = static_cast<const uint16_t*>(p.k);

@@ -357,29 +357,6 @@ __device__ __forceinline__ int seq_of(const int* pref, int B, long long hr_count
   return lo;
 }
 
-// Wave-wide inclusive sum / maximum (x >= 0) of one int per lane through DPP
-// row shifts and row broadcasts: lane l gets the result over lanes 0..l, with
-// no LDS round trip.
-__device__ __forceinline__ int wave_incl_sum(int x) {
-  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, false);  // row_shr:1
-  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, false);  // row_shr:2
-  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, false);  // row_shr:4
-  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, false);  // row_shr:8
-  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, false);  // row_bcast:15
-  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, false);  // row_bcast:31
-  return x;
-}
-__device__ __forceinline__ int wave_incl_max(int x) {
-  x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, false));
-  x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, false));
-  x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, false));
-  x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, false));
-  x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, false));
-  x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, false));
-  return x;
-}
-__device__ __forceinline__ int lane63(int x) { return __builtin_amdgcn_readlane(x, 63); }
-
 // floor(a / b) for 0 <= a < 2^53, b >= 1: the correctly rounded double
 // quotient truncates to the exact one (64-bit integer division would expand
 // to a long instruction sequence).
