@@ -64,7 +64,11 @@ static_assert(kChunk % (4 * kThreads) == 0, "every thread of a race chunk takes 
 // 45.9 with 3 pieces, 48.4 with whole rows), with every row read 352 (whole
 // rows: 57.7 us; 2 pieces were slower).
 constexpr int kMaxSplit = 8;
-constexpr int kStatGroups = 512;
+// Greedy rows (an argmax; no race follows, so the pieces' tail is the call's
+// end): 768 groups, gamma = 5, us per call with 512 / 768 / 1024: B = 16 32.8 /
+// 29.7 / 32.0, B = 24 47.5 / 39.0 / 40.4, B = 32 49.4 / 43.4 / 43.9; larger batches
+// the same.
+constexpr int kStatGroups = 512, kStatGroupsGreedy = 768;
 constexpr int kVecPerThread = kChunk / 4 / kThreads;
 // The race streams its chunk in steps of kRaceStep float4 of p, q and E per
 // thread, the next step's loads in flight while one is raced, and races the
@@ -1217,7 +1221,7 @@ int spv::verify_sample_impl(const float* target, const float* draft, int is_prob
   const bool unit = a.tf == 1.0f;
   if (!is_probs) {
     const int rows = B * (draft_stats ? gamma + 1 : 2 * gamma + 1);
-    a.split = std::max(1, std::min(kMaxSplit, kStatGroups / rows));
+    a.split = std::max(1, std::min(kMaxSplit, (greedy ? kStatGroupsGreedy : kStatGroups) / rows));
     const dim3 grid(rows * a.split);
     if (greedy)
       hipLaunchKernelGGL((row_stats_kernel<IN_GREEDY, true>), grid, dim3(kThreads), 0, s, a, cm, ws);
