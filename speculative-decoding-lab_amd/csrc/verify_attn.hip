@@ -71,6 +71,7 @@ struct AttnParams {
   int pages_per_split, max_splits, nrg, rows_per_group;
   int max_pages;     // ceil(max_ctx / block_size): no table entry beyond it is read
   float scale_log2;  // softmax scale * log2(e)
+  float piece_root;  // of min_piece, by the page type
   int* plan;         // MFMA path: the round's plan (written by attn_plan_kernel, read by planned calls)
   // Planned calls over 16-bit pages: this layer's chunk (B, C, Hkv, d) and the
   // pool row of each of its tokens, to be written before it is attended
@@ -280,19 +281,24 @@ __host__ __device__ constexpr int piece_cost(int d, int kt) {
 constexpr int kMfmaThreads = 512;
 // The smallest piece of the equal-pieces split, in pages, for a longest
 // context of `maxnp` pages: cutting finer than fills the workgroups' waves
-// only adds partials. A piece of 16 pages gives each of the eight waves two; a
-// segment of np pages in pieces of P costs about t_page P / 8 of walk and
-// t_merge np / (8 P) of the last arriver's merge (kMergeChunk slots a round
-// trip), least near P = sqrt(np t_merge / t_page) -- 2 sqrt(np) measured.
+// only adds partials. A segment of np pages in pieces of P costs about
+// t_page P / 8 of walk (eight waves) and t_merge np / (8 P) of the last
+// arriver's merge (kMergeChunk slots a round trip), least near
+// P = sqrt(np t_merge / t_page): 1.5 sqrt(np) measured over 16-bit pages, 2 over
+// the smaller fp8 pages; and never below 12.
 // Without the bound a small batch was cut into pieces of one or two pages and
-// merges of up to 256 slots (planned calls, us, without / with): batch 8 of 64
-// to 1,024 keys, 12/2 heads of 128, 30.8 / 14.5; one sequence of 4,096 keys
-// 40.1 / 15.8, of 16,384 66.6 / 28.5; two of 32,768 over fp8 pages, 14/2
-// heads of 64, 45.9 / 30.4; one-row decode of 1,000 keys 20.5 / 6.4. (Floors
-// of 8 and 32 pages: 14.3 and 14.4 at the first shape, 7.4 and 7.8 at the
-// last; 1.4 sqrt and 2.8 sqrt: 28.0 and 29.8 at 16,384 keys.) Batches that
-// fill the grid with longer pieces than this are cut as before.
-__device__ __forceinline__ int min_piece(int maxnp) { return max(16, (int)(2.f * __builtin_sqrtf((float)maxnp))); }
+// merges of up to 256 slots (planned calls, us, without / with 16 and 2 sqrt):
+// batch 8 of 64 to 1,024 keys, 12/2 heads of 128, 30.8 / 14.5; one sequence of
+// 4,096 keys 40.1 / 15.8; one-row decode of 1,000 keys 20.5 / 6.4. Whole
+// measurements with (16, 2 sqrt) / (12, 1.5 sqrt) / (12, sqrt): a 28-layer round of
+// the first batch, fp16, 534 / 512 / 514 us; four planned layers of one sequence
+// of 4,096 keys 82.8 / 79.9 / 86.3, of 16,384 118.0 / 115.3 / 128.4; two of 32,768
+// over fp8 pages, 14/2 heads of 64, two layers with their appends 80.0 / 83.5 /
+// 95.2. Batches that fill the grid with longer pieces than this are cut as before.
+__host__ __device__ constexpr float piece_root(int kt) { return kt == SPV_FP8E4M3 ? 2.f : 1.5f; }
+__device__ __forceinline__ int min_piece(int maxnp, float root) {
+  return max(12, (int)(root * __builtin_sqrtf((float)maxnp)));
+}
 // O^T tiles combined per LDS round: as many as fit beside the other buffers
 // (the slots take 8 waves x 16 * nt rows x 64 B per tile). With four query
 // tiles: all four of head_dim 64 in one round (long context 2 us faster than
@@ -420,7 +426,7 @@ __device__ void build_plan(const AttnParams& p, int* s_pref, int* s_kpref, int* 
     auto pages_of = [&](int b) { return one ? np1 : s_pref[b + 1] - s_pref[b]; };
     const long long T = HR * carry;
     int P = HR * p.B >= nw ? maxnp
-                           : (int)min((long long)maxnp, max((long long)min_piece(maxnp), div_floor(T + nw - 1, nw)));
+                           : (int)min((long long)maxnp, max((long long)min_piece(maxnp, p.piece_root), div_floor(T + nw - 1, nw)));
     int npieces;
     for (;;) {
       const float rP = __builtin_amdgcn_rcpf((float)P);
@@ -1977,6 +1983,7 @@ int spv::verify_attn_impl(void* out, const void* q, int q_dtype, const void* k_p
   p.rows_per_group = pl.rows_per_group;
   p.max_pages = (max_ctx + block_size - 1) / block_size;
   p.scale_log2 = scale * kLog2e;
+  p.piece_root = piece_root(kv_dtype);
   // A round's plan serves MFMA calls only (the VALU path has no prologue to skip).
   if (pl.plannable() && plan) p.plan = static_cast<int*>(const_cast<void*>(plan));
   // A chunk still to be written: by the planned kernels over 16-bit pages
@@ -2095,6 +2102,7 @@ int spv_verify_attn_plan(const int32_t* block_tables, int32_t max_blocks_per_seq
   p.nrg = pl.nrg;
   p.rows_per_group = pl.rows_per_group;
   p.max_pages = (max_ctx + block_size - 1) / block_size;
+  p.piece_root = piece_root(kv_dtype);
   p.plan = static_cast<int*>(plan);
   launch_plan(p, head_dim, kv_dtype, (hipStream_t)stream);
   SPV_CHECK_LAUNCH();

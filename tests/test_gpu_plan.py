@@ -139,10 +139,12 @@ def test_plan_reports_unwritten_keys(cuda):
 
 
 @pytest.mark.parametrize("B,Hq,Hkv,d,C,lo,hi", [
-    (1, 12, 2, 128, 6, 250, 250),      # one page less than, or exactly, one smallest piece (16 pages)
-    (1, 12, 2, 128, 6, 251, 251),      # one page more: two pieces
-    (2, 14, 2, 64, 1, 1017, 1030),     # the floor meets 2 sqrt(pages) at 64 pages, one row
-    (1, 12, 2, 128, 4, 16000, 16000),  # pieces of 63 pages: 16 partials, two merge round trips
+    (1, 12, 2, 128, 6, 186, 186),      # exactly one smallest piece (12 pages)
+    (1, 12, 2, 128, 6, 187, 187),      # one page more: two pieces
+    (1, 12, 2, 128, 6, 250, 250),
+    (1, 12, 2, 128, 6, 251, 251),
+    (2, 14, 2, 64, 1, 1017, 1030),     # the floor meets 1.5 sqrt(pages) at 64 pages, one row
+    (1, 12, 2, 128, 4, 16000, 16000),  # pieces of 47 pages: 22 partials, three merge round trips
     (3, 16, 2, 128, 9, 3, 9000),       # four query tiles and two row groups, one context far longer
 ])
 def test_smallest_piece_of_the_equal_split(cuda, B, Hq, Hkv, d, C, lo, hi):
