@@ -28,6 +28,7 @@
 // a (sequence, kv head, row group, split) grid and its own merge kernel.
 #include <math.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include <hip/hip_ext.h>
@@ -706,7 +707,8 @@ __device__ __forceinline__ int xswz(int r) { return ((r >> 1) ^ (r >> 3)) & 3; }
 // it: its first piece and the block ids of each wave's first page come in one
 // load, so the page walk starts one round trip after launch.
 // AP: a planned call that writes its chunk's keys and values first.
-template <int NT, int D, int QT, bool BAL, int KT, bool PL, bool AP = false>
+// HL: fp16 pages take P in two halves (see compute_page).
+template <int NT, int D, int QT, bool BAL, int KT, bool PL, bool AP = false, bool HL = true>
 __global__ __launch_bounds__(kMfmaThreads, 1) void attn_mfma_kernel(AttnParams p) {
   constexpr bool kFp8 = KT == SPV_FP8E4M3;
   // fp16 pages take fp16 queries (S^T and P V on the fp16 MFMAs); bf16 and
@@ -1132,10 +1134,12 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void attn_mfma_kernel(AttnParams p
       // P vf stays in fp16's normal range; an all-zero block (sv = 0) has
       // P vf = 0. bf16 pages, and fp8 pages in the
       // head_dim-128 kernels with four query tiles (no register to spare),
-      // take P V in bf16 hi + lo. fp16 pages take P V in fp16 with V^T as it
-      // is (vf = 1): P < 2^kSlack, and P in fp16 keeps 11 bits, the precision
-      // of the fp16 output.
-      constexpr bool h16 = (kFp8 && !(NT == 4 && D == 128)) || kF16;
+      // take P V in bf16 hi + lo. fp16 pages take P V in fp16 hi + lo, too
+      // (HL): P in one fp16 (11 bits) added to the fp16 output's own rounding,
+      // error against float64 2.5e-4 to 2.7e-4, growing with the keys that
+      // share a reference maximum, against 2.1e-4; and the wider MFMA is no
+      // slower (a 28-layer round of 8 sequences, 12/2 heads of 128, 517 -> 502 us).
+      constexpr bool h16 = (kFp8 && !(NT == 4 && D == 128)) || (kF16 && !HL);
       float vf = 1.f, vsc = 1.f;
       int vc = 0;
       if constexpr (h16 && kFp8) {
@@ -1373,29 +1377,37 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void attn_mfma_kernel(AttnParams p
             for (int nt = 0; nt < NT; ++nt) o[mt][nt] *= o_up;
         }
       } else {
-        bf16x8_t pf[NT];
+        // P = hi + lo in the pages' 16-bit type (bf16; fp16 for fp16 pages)
+        using V2 = std::conditional_t<kF16, f16x2_t, bf16x2_t>;
+        uint4 pf[NT];
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
           float e[4];
           p_tile(nt, e);
-          // P = hi + lo, both bf16: slots 0..3 carry hi, 4..7 lo of the same keys,
-          // so one 16x16x32 MFMA against {V, V} accumulates P V to ~16 bits.
-          const bf16x2_t h01 = __builtin_convertvector(f32x2_t{e[0], e[1]}, bf16x2_t);
-          const bf16x2_t h23 = __builtin_convertvector(f32x2_t{e[2], e[3]}, bf16x2_t);
+          // slots 0..3 carry hi, 4..7 lo of the same keys, so one 16x16x32 MFMA
+          // against {V, V} accumulates P V to ~16 bits (bf16; ~22 in fp16).
+          const V2 h01 = __builtin_convertvector(f32x2_t{e[0], e[1]}, V2);
+          const V2 h23 = __builtin_convertvector(f32x2_t{e[2], e[3]}, V2);
           const f32x2_t r01 = f32x2_t{e[0], e[1]} - __builtin_convertvector(h01, f32x2_t);
           const f32x2_t r23 = f32x2_t{e[2], e[3]} - __builtin_convertvector(h23, f32x2_t);
-          pf[nt] = __builtin_bit_cast(
-              bf16x8_t, make_uint4(__builtin_bit_cast(uint32_t, h01), __builtin_bit_cast(uint32_t, h23),
-                                   pack2_bf16(r01[0], r01[1]), pack2_bf16(r23[0], r23[1])));
+          pf[nt] = make_uint4(__builtin_bit_cast(uint32_t, h01), __builtin_bit_cast(uint32_t, h23),
+                              __builtin_bit_cast(uint32_t, __builtin_convertvector(r01, V2)),
+                              __builtin_bit_cast(uint32_t, __builtin_convertvector(r23, V2)));
         }
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
           // {V^T, V^T}: the same keys in both halves of the k-slots.
           const uint2 vv = vfrag(mt);
-          const bf16x8_t va = __builtin_bit_cast(bf16x8_t, make_uint4(vv.x, vv.y, vv.x, vv.y));
+          const uint4 va = make_uint4(vv.x, vv.y, vv.x, vv.y);
 #pragma unroll
-          for (int nt = 0; nt < NT; ++nt)
-            o[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, pf[nt], o[mt][nt], 0, 0, 0);
+          for (int nt = 0; nt < NT; ++nt) {
+            if constexpr (kF16)
+              o[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, va),
+                                                                 __builtin_bit_cast(f16x8_t, pf[nt]), o[mt][nt], 0, 0, 0);
+            else
+              o[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, va),
+                                                                  __builtin_bit_cast(bf16x8_t, pf[nt]), o[mt][nt], 0, 0, 0);
+          }
         }
       }
     };
@@ -1835,7 +1847,22 @@ void launch_mfma_mode(const AttnParams& p, int nt, hipStream_t s, dim3 grid, siz
     case 2: launch_attn(attn_mfma_kernel<2, D, QT, BAL, KT, PL, AP>, grid, blk, smem, s, true, true, p); break;
     case 3: launch_attn(attn_mfma_kernel<3, D, QT, BAL, KT, PL, AP>, grid, blk, smem, s, true, true, p); break;
     default:  // four query tiles: planned only at head_dim 64 (Plan::plannable)
-      launch_attn(attn_mfma_kernel<4, D, QT, BAL, KT, PL && D != 128, AP && D != 128>, grid, blk, smem, s, true, true, p);
+      if constexpr (D == 128 && KT == SPV_F16) {
+        // No register to spare here: the second half of P costs 2-4% (16/2 heads
+        // of 128, chunk 7, us per call: 32 sequences of 256 to 4,096 keys 27.9 ->
+        // 29.0, 128 of 512 to 8,192 101 -> 103). It is taken where the smallest
+        // piece sets the split -- a batch too short to fill the grid with longer
+        // ones -- whose waves share a reference maximum over more keys than a
+        // finer cut's would.
+        const int mp = p.max_pages;
+        const long long least = std::max(12, (int)(p.piece_root * sqrtf((float)mp)));
+        if (BAL || (long long)p.Hkv * p.nrg * p.B * mp > least * grid.x)
+          launch_attn(attn_mfma_kernel<4, D, QT, BAL, KT, false, false, false>, grid, blk, smem, s, true, true, p);
+        else
+          launch_attn(attn_mfma_kernel<4, D, QT, false, KT, false>, grid, blk, smem, s, true, true, p);
+      } else {
+        launch_attn(attn_mfma_kernel<4, D, QT, BAL, KT, PL && D != 128, AP && D != 128>, grid, blk, smem, s, true, true, p);
+      }
       break;
   }
 }
