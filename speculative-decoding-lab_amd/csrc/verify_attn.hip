@@ -28,7 +28,6 @@
 // a (sequence, kv head, row group, split) grid and its own merge kernel.
 #include <math.h>
 
-#include <algorithm>
 #include <type_traits>
 
 #include <hip/hip_ext.h>
@@ -398,9 +397,15 @@ __device__ __forceinline__ int ceil_div(int a, int P, float rP) {
 // segment costs its pages plus `piece_cost` pages for the set-up, combine and
 // merge of a piece, so s_pref[b] sums (pages + piece_cost) -- and the search
 // and s_kpref are skipped.
+// `s_coarse` (kernels that take P in two halves where the smallest piece sets the
+// split, kPick): *s_coarse gets whether it does. Up to 1.25 times the even share it
+// does not there: the second half would cost more than the longer piece saves
+// (fp16, 16/2 heads of 128, us per call, even share and one half / smallest piece
+// and two: 24 sequences, 20 pages for an even 19, 27.1 / 28.3; at 1.33, 1.44 and
+// 1.45 times 26.3 / 26.0, 28.7 / 28.2 and 24.7 / 23.5).
 template <int BS, bool BAL>
 __device__ void build_plan(const AttnParams& p, int* s_pref, int* s_kpref, int* s_sid, int* s_start, long long HR,
-                           int nw, int piece_cost) {
+                           int nw, int piece_cost, int* s_coarse = nullptr) {
   if (threadIdx.x < 64) {
     const int lane = threadIdx.x;
     const bool one = p.B <= 64;  // the common case keeps every count in a register
@@ -426,8 +431,14 @@ __device__ void build_plan(const AttnParams& p, int* s_pref, int* s_kpref, int* 
     if constexpr (!BAL) {
     auto pages_of = [&](int b) { return one ? np1 : s_pref[b + 1] - s_pref[b]; };
     const long long T = HR * carry;
-    int P = HR * p.B >= nw ? maxnp
-                           : (int)min((long long)maxnp, max((long long)min_piece(maxnp, p.piece_root), div_floor(T + nw - 1, nw)));
+    const long long even = div_floor(T + nw - 1, nw);
+    long long least = min_piece(maxnp, p.piece_root);
+    if (s_coarse) {
+      const bool coarse = HR * p.B < nw && 4 * least > 5 * even;
+      if (!coarse) least = even;
+      if (lane == 0) *s_coarse = coarse;
+    }
+    int P = HR * p.B >= nw ? maxnp : (int)min((long long)maxnp, max(least, even));
     int npieces;
     for (;;) {
       const float rP = __builtin_amdgcn_rcpf((float)P);
@@ -707,8 +718,7 @@ __device__ __forceinline__ int xswz(int r) { return ((r >> 1) ^ (r >> 3)) & 3; }
 // it: its first piece and the block ids of each wave's first page come in one
 // load, so the page walk starts one round trip after launch.
 // AP: a planned call that writes its chunk's keys and values first.
-// HL: fp16 pages take P in two halves (see compute_page).
-template <int NT, int D, int QT, bool BAL, int KT, bool PL, bool AP = false, bool HL = true>
+template <int NT, int D, int QT, bool BAL, int KT, bool PL, bool AP = false>
 __global__ __launch_bounds__(kMfmaThreads, 1) void attn_mfma_kernel(AttnParams p) {
   constexpr bool kFp8 = KT == SPV_FP8E4M3;
   // fp16 pages take fp16 queries (S^T and P V on the fp16 MFMAs); bf16 and
@@ -727,6 +737,10 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void attn_mfma_kernel(AttnParams p
   static_assert(QT == (kF32 ? SPV_F32 : kF16 ? SPV_F16 : SPV_BF16), "query type follows the page type");
   using QE = std::conditional_t<kF32, float, uint16_t>;
   constexpr int kQV = 16 / (int)sizeof(QE);  // query elements in 16 bytes
+  // fp16 pages in these kernels: P in one half, or (kPick) in two where the split is
+  // `coarse` (see compute_page).
+  constexpr bool kHalf = kF16 && NT == 4 && D == 128, kPick = kHalf && !BAL;
+  bool coarse = false;
   // Block ids (and fp8 scales) of a window per lane, or per page from LDS
   // (see the page walk).
   constexpr bool kLaneIds = D == 64 || (NT <= 2 && !(kF32 && NT == 2)) || (NT == 3 && PL);
@@ -804,8 +818,10 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void attn_mfma_kernel(AttnParams p
     sid = word(H_SID);
     first_id = __builtin_amdgcn_readlane(hv, H_IDS + w);  // this wave's first page
   } else {
-    build_plan<BS, BAL>(p, s_pref, s_kpref, s_sid, s_start, HR, nw, KPC);
+    __shared__ int s_coarse;
+    build_plan<BS, BAL>(p, s_pref, s_kpref, s_sid, s_start, HR, nw, KPC, kPick ? &s_coarse : nullptr);
     if (s_pref[p.B] == 0) return;
+    if constexpr (kPick) coarse = uni(s_coarse) != 0;
     const ShareRange r = share_range<BAL>(s_pref, s_kpref, p.B, HR, KPC, nw, wg);
     x_begin = r.x_begin;
     x_stop = r.x_stop;
@@ -1134,12 +1150,20 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void attn_mfma_kernel(AttnParams p
       // P vf stays in fp16's normal range; an all-zero block (sv = 0) has
       // P vf = 0. bf16 pages, and fp8 pages in the
       // head_dim-128 kernels with four query tiles (no register to spare),
-      // take P V in bf16 hi + lo. fp16 pages take P V in fp16 hi + lo, too
-      // (HL): P in one fp16 (11 bits) added to the fp16 output's own rounding,
-      // error against float64 2.5e-4 to 2.7e-4, growing with the keys that
-      // share a reference maximum, against 2.1e-4; and the wider MFMA is no
-      // slower (a 28-layer round of 8 sequences, 12/2 heads of 128, 517 -> 502 us).
-      constexpr bool h16 = (kFp8 && !(NT == 4 && D == 128)) || (kF16 && !HL);
+      // take P V in bf16 hi + lo. fp16 pages take P V in fp16 hi + lo, too: P in
+      // one fp16 (11 bits) adds to the fp16 output's own rounding, error against
+      // float64 2.4e-4 to 2.8e-4, growing with the keys that share a reference
+      // maximum (the maximum itself is exact in P), against 2.1e-4; and the wider
+      // MFMA is no slower (a 28-layer round of 8 sequences, 12/2 heads of 128,
+      // 517 -> 502 us). In the head_dim-128 kernels with four query tiles (no
+      // register to spare, 3-4% slower) P stays in one half where the batch fills
+      // the grid, cut as finely as ever; where the smallest piece sets the split
+      // (`coarse`, from the batch's own pages, not from the caller's max_ctx) the
+      // second half is multiplied after the first, two tiles at a time: one
+      // context of 4,096 keys and fifteen of 256, 16/2 heads, chunk 7, error 2.7e-4
+      // with one half, 2.1e-4 with two (24.5 and 26.2 us per call); a batch that
+      // fills the grid pays 0.2-0.4 us for the test.
+      constexpr bool h16 = (kFp8 && !(NT == 4 && D == 128)) || kHalf;
       float vf = 1.f, vsc = 1.f;
       int vc = 0;
       if constexpr (h16 && kFp8) {
@@ -1358,16 +1382,36 @@ __global__ __launch_bounds__(kMfmaThreads, 1) void attn_mfma_kernel(AttnParams p
         }
         // P as fp16 (16x16x16: lane l holds keys 4 (l / 16) .. + 3 of column
         // l % 16, the accumulator layout of S^T; V^T the same keys of dim l % 16).
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-          float e[4];
-          p_tile(nt, e);
+        auto add_pv = [&](int nt, f16x2_t p01, f16x2_t p23) {
           const f16x4_t pv = __builtin_bit_cast(
-              f16x4_t, make_uint2(__builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{e[0], e[1]}, f16x2_t)),
-                                  __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{e[2], e[3]}, f16x2_t))));
+              f16x4_t, make_uint2(__builtin_bit_cast(uint32_t, p01), __builtin_bit_cast(uint32_t, p23)));
 #pragma unroll
           for (int mt = 0; mt < MT; ++mt)
             o[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(f16x4_t, vfrag(mt)), pv, o[mt][nt], 0, 0, 0);
+        };
+        constexpr int kNP = kPick ? 2 : 1;
+#pragma unroll
+        for (int n0 = 0; n0 < NT; n0 += kNP) {
+          f32x2_t e01[kNP], e23[kNP];
+          f16x2_t h01[kNP], h23[kNP];
+#pragma unroll
+          for (int k = 0; k < kNP; ++k) {
+            float e[4];
+            p_tile(n0 + k, e);
+            e01[k] = f32x2_t{e[0], e[1]};
+            e23[k] = f32x2_t{e[2], e[3]};
+            h01[k] = __builtin_convertvector(e01[k], f16x2_t);
+            h23[k] = __builtin_convertvector(e23[k], f16x2_t);
+            add_pv(n0 + k, h01[k], h23[k]);
+          }
+          if constexpr (kPick) {
+            if (coarse) {
+#pragma unroll
+              for (int k = 0; k < kNP; ++k)
+                add_pv(n0 + k, __builtin_convertvector(e01[k] - __builtin_convertvector(h01[k], f32x2_t), f16x2_t),
+                       __builtin_convertvector(e23[k] - __builtin_convertvector(h23[k], f32x2_t), f16x2_t));
+            }
+          }
         }
         if (vc) {
           const float o_up = __builtin_bit_cast(float, (uint32_t)(127 + vc) << 23);
@@ -1847,22 +1891,7 @@ void launch_mfma_mode(const AttnParams& p, int nt, hipStream_t s, dim3 grid, siz
     case 2: launch_attn(attn_mfma_kernel<2, D, QT, BAL, KT, PL, AP>, grid, blk, smem, s, true, true, p); break;
     case 3: launch_attn(attn_mfma_kernel<3, D, QT, BAL, KT, PL, AP>, grid, blk, smem, s, true, true, p); break;
     default:  // four query tiles: planned only at head_dim 64 (Plan::plannable)
-      if constexpr (D == 128 && KT == SPV_F16) {
-        // No register to spare here: the second half of P costs 2-4% (16/2 heads
-        // of 128, chunk 7, us per call: 32 sequences of 256 to 4,096 keys 27.9 ->
-        // 29.0, 128 of 512 to 8,192 101 -> 103). It is taken where the smallest
-        // piece sets the split -- a batch too short to fill the grid with longer
-        // ones -- whose waves share a reference maximum over more keys than a
-        // finer cut's would.
-        const int mp = p.max_pages;
-        const long long least = std::max(12, (int)(p.piece_root * sqrtf((float)mp)));
-        if (BAL || (long long)p.Hkv * p.nrg * p.B * mp > least * grid.x)
-          launch_attn(attn_mfma_kernel<4, D, QT, BAL, KT, false, false, false>, grid, blk, smem, s, true, true, p);
-        else
-          launch_attn(attn_mfma_kernel<4, D, QT, false, KT, false>, grid, blk, smem, s, true, true, p);
-      } else {
-        launch_attn(attn_mfma_kernel<4, D, QT, BAL, KT, PL && D != 128, AP && D != 128>, grid, blk, smem, s, true, true, p);
-      }
+      launch_attn(attn_mfma_kernel<4, D, QT, BAL, KT, PL && D != 128, AP && D != 128>, grid, blk, smem, s, true, true, p);
       break;
   }
 }

@@ -35,3 +35,33 @@ def test_error_against_float64(cuda, B, C, Hq, Hkv, d, hi, bound):
     want = ref_attn.extend_attention_dense(q.float(), [k.float() for k in keys], [v.float() for v in values], lens, Hq)
     err = float((out.cpu().double() - want.double()).norm() / want.double().norm())
     assert err <= bound, err
+
+
+@pytest.mark.parametrize("B,C,lo,hi", [
+    (16, 7, 256, 4096),   # even share 4 pages, smallest piece 24
+    (16, 7, 64, 4096),
+    (20, 8, 700, 3000),   # even share 9, smallest piece 20
+    (9, 7, 16, 12000),    # smallest piece 41
+])
+def test_ragged_batches_with_four_tiles_at_128(cuda, B, C, lo, hi):
+    """One long context among short ones: the batch's own pages leave the grid
+    unfilled, though B times the longest context would fill it. The pieces are the
+    smallest ones, so P is in two halves; a looser max_ctx changes nothing."""
+    lens = [lo] * (B // 2) + [hi] + [lo] * (B - 1 - B // 2)
+    gpu, keys, values = _dense_pool(cuda, lens, C, 2, 128, 16, torch.float16, seed=hi)
+    q = torch.randn(B, C, 16, 128, generator=torch.Generator().manual_seed(B + lo)).to(torch.float16)
+    out = verify_attention(q.to(cuda), gpu, 0, list(range(B)), lens, hi + C)
+    want = ref_attn.extend_attention_dense(q.float(), [k.float() for k in keys], [v.float() for v in values], lens, 16)
+    err = float((out.cpu().double() - want.double()).norm() / want.double().norm())
+    assert err <= 2.2e-4, err  # the output's rounding, 2.0e-4 to 2.1e-4; one half of P would add 1.2e-4 or more in quadrature
+    for more in (1.5, 4):
+        assert torch.equal(verify_attention(q.to(cuda), gpu, 0, list(range(B)), lens, int(hi * more)), out), more
+
+
+def test_loose_max_ctx_leaves_a_full_grid_alone(cuda):
+    """One half of P (the batch fills the grid): the same bits whatever max_ctx."""
+    lens, C = [300 + 97 * b for b in range(28)], 7
+    gpu, _, _ = _dense_pool(cuda, lens, C, 2, 128, 16, torch.float16, seed=3)
+    q = torch.randn(28, C, 16, 128, generator=torch.Generator().manual_seed(4)).to(torch.float16).to(cuda)
+    out = verify_attention(q, gpu, 0, list(range(28)), lens, max(lens) + C)
+    assert torch.equal(verify_attention(q, gpu, 0, list(range(28)), lens, 20000), out)
