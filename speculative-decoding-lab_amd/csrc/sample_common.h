@@ -243,9 +243,10 @@ inline float temperature_divisor(float T) { return (float)((double)T > kEps ? (d
 // row is off by up to ~1e-5, and the cumulative sum rounds each entry.
 constexpr double kTopPWindow = 5e-5;
 
-// Larger x, larger key; NaN above everything (torch.topk ranks NaN first).
+// Larger x, larger key; NaN above everything (torch.topk ranks NaN first). Both
+// zeros have the key of +0.0: they are equal to the filters' float comparisons.
 __device__ __forceinline__ uint32_t order_key(float x) {
-  const uint32_t u = __float_as_uint(x);
+  const uint32_t u = __float_as_uint(x + 0.f);
   if (x != x) return 0xffffffffu;
   return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }

@@ -267,3 +267,28 @@ def test_filtered_sampler_rows_the_short_form_leaves(cuda, odd):
     assert torch.equal(got.accept_len, want.accept_len)
     assert torch.equal(got.out_tokens, want.out_tokens)
     assert torch.equal(got.flags, want.flags)
+
+
+@pytest.mark.parametrize("T", [1.0, 0.7])
+@pytest.mark.parametrize("top_k,above", [(40, 30), (600, 590)])  # the short form, the general path
+def test_both_zeros_tie_at_the_kth_value(cuda, T, top_k, above):
+    """The k-th value is +0.0: the float comparison drops neither zero, so a token
+    at -0.0 stays and can be drawn."""
+    vocab, B, gamma = 3000, 3, 2
+    g = torch.Generator().manual_seed(top_k)
+    z = -torch.rand(B, gamma + 1, vocab, generator=g) - 0.5
+    perm = torch.randperm(vocab, generator=g)
+    up, plus, minus = perm[:above], perm[above:above + 20], perm[above + 20:above + 45]
+    z[..., up] = torch.rand(B, gamma + 1, above, generator=g) * 0.5
+    z[..., plus], z[..., minus] = 0.0, -0.0
+    want = S.filter_logits(z, T, top_k, 1.0)
+    assert bool(torch.isfinite(want[..., minus]).all()) and int(torch.isfinite(want[0, 0]).sum()) == above + 45
+    assert torch.equal(_hip.filter_rows(z.to(cuda), T, top_k, 1.0).cpu(), want)
+    draft = z[:, :gamma].contiguous()
+    x = up[torch.arange(B * gamma).reshape(B, gamma)].int()
+    u = torch.zeros(B, gamma)
+    noise = torch.empty(B, vocab).exponential_(1, generator=g).clamp_min_(0.1)
+    noise[:, minus[3]] = 1e-6  # the bonus draw goes to a token at -0.0
+    got = es.verify_sample(z.to(cuda), draft.to(cuda), x.to(cuda), u.to(cuda), noise.to(cuda), T, top_k=top_k)
+    assert got.accepted_lists() == S.verify_from_logits(z, draft, x, u, noise, T, top_k, 1.0)
+    assert all(t[-1] == int(minus[3]) for t in got.accepted_lists())
