@@ -230,9 +230,12 @@ class Workspace:
     that share a buffer must be ordered: giving each stream its own buffer
     keeps calls on two streams from racing on counters and partials. A buffer
     replaced by a larger one is kept alive for the life of the object, since a
-    HIP graph captured earlier may still point at it."""
+    HIP graph captured earlier may still point at it. ``factor``: a buffer is
+    replaced by one at least that many times as large; with 2 the replaced ones
+    together stay below the one in use, however slowly a batch grows."""
 
-    def __init__(self) -> None:
+    def __init__(self, factor: int = 1) -> None:
+        self._factor = factor
         self._bufs: dict = {}
         self._retired: list = []
 
@@ -246,9 +249,11 @@ class Workspace:
         key = self._key(device, stream)
         buf = self._bufs.get(key)
         if buf is None or buf.numel() < nbytes:
+            size = max(int(nbytes), 256)
             if buf is not None:
                 self._retired.append(buf)
-            buf = torch.zeros(max(int(nbytes), 256), dtype=torch.uint8, device=device)
+                size = max(size, self._factor * buf.numel())
+            buf = torch.zeros(size, dtype=torch.uint8, device=device)
             self._bufs[key] = buf
         return buf
 

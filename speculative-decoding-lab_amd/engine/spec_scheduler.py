@@ -41,7 +41,7 @@ from .attention import VerifyPlan, append_verify_attention, verify_attention
 from .kv import PagedKVCache, WritePlan
 
 _workspace = _hip.Workspace()
-_filter_workspace = _hip.Workspace()
+_filter_workspace = _hip.Workspace(factor=2)  # lists of about 0.9 MB per sequence (gamma 5, V = 151,936)
 _draft_workspace = _hip.Workspace()
 
 
