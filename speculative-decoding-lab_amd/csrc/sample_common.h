@@ -173,9 +173,6 @@ struct DecideArgs {
   int B, gamma, V, is_probs, greedy, decide_only;
   int split;  // pieces per statistics row
   float tf;
-  const int32_t* need;   // (B) or null: the sequences with need[b] == 0 are skipped
-  const int32_t* amb_t;  // (B, gamma + 1) or null: window counts of the filtered rows
-  const int32_t* amb_d;  // (B, gamma)
 };
 
 struct CommitArgs {
