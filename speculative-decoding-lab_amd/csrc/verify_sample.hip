@@ -64,11 +64,22 @@ static_assert(kChunk % (4 * kThreads) == 0, "every thread of a race chunk takes 
 // 45.9 with 3 pieces, 48.4 with whole rows), with every row read 352 (whole
 // rows: 57.7 us; 2 pieces were slower).
 constexpr int kMaxSplit = 8;
+constexpr int kStatGroups = 512;
 // Greedy rows (an argmax; no race follows, so the pieces' tail is the call's
-// end): 768 groups, gamma = 5, us per call with 512 / 768 / 1024: B = 16 32.8 /
-// 29.7 / 32.0, B = 24 47.5 / 39.0 / 40.4, B = 32 49.4 / 43.4 / 43.9; larger batches
-// the same.
-constexpr int kStatGroups = 512, kStatGroupsGreedy = 768;
+// end): up to 768 groups where that makes at most five pieces of a row, each of
+// 15,000 values or more (rows that are not whole float4, read one value at a time,
+// whatever their length). us per call in a graph, floor(512 / rows) pieces / these
+// / floor(768 / rows): V = 151,936, 132 rows 27.1 / 25.7 / 25.7, 176 32.1 / 28.3 /
+// 28.3, 264 46.2 / 35.3 / 35.3, 88 23.0 / 23.0 / 23.3; V = 32,000, 112 rows 15.2 /
+// 15.2 / 16.9, 176 16.9 / 16.9 / 18.2, 264 19.4 / 17.0 / 17.0; V = 50,257, 176 rows
+// 40.8 / 29.4 / 29.4, 88 19.5 / 19.5 / 20.1. Beyond 768 rows there is one piece.
+constexpr int kStatGroupsGreedy = 768, kGreedyPieces = 5, kGreedyPiece = 15000;
+inline int stat_pieces(int rows, int V, bool greedy) {
+  int n = kStatGroups / rows;
+  if (greedy)
+    n = std::max(n, std::min({kGreedyPieces, kStatGroupsGreedy / rows, (V & 3) ? kGreedyPieces : V / kGreedyPiece}));
+  return std::max(1, std::min(kMaxSplit, n));
+}
 constexpr int kVecPerThread = kChunk / 4 / kThreads;
 // The race streams its chunk in steps of kRaceStep float4 of p, q and E per
 // thread, the next step's loads in flight while one is raced, and races the
@@ -1235,7 +1246,7 @@ int spv::verify_sample_impl(const float* target, const float* draft, int is_prob
   if (filt && (is_probs || greedy || !unit)) return SPV_ERR_ARG;  // filtered rows are sampled at T = 1
   if (!is_probs) {
     const int rows = B * (draft_stats ? gamma + 1 : 2 * gamma + 1);
-    a.split = std::max(1, std::min(kMaxSplit, (greedy ? kStatGroupsGreedy : kStatGroups) / rows));
+    a.split = stat_pieces(rows, V, greedy);
     const dim3 grid(rows * a.split);
     if (greedy)
       hipLaunchKernelGGL((row_stats_kernel<IN_GREEDY, true, false>), grid, dim3(kThreads), 0, s, a, cm, ws, fa);

@@ -448,3 +448,33 @@ def test_exact_race_visits_every_contending_chunk(cuda, V, a, b, reject):
         assert res.accepted_lists() == [[token] if reject else [7, token]]
         assert res.accepted_lists() == S.batch_accept_noise(p, q, x, u, e)
         assert res.flags.tolist() == [flag]
+
+
+@pytest.mark.parametrize("B,gamma,V", [
+    (8, 5, 32000),    # five pieces, by the sampled rule
+    (16, 5, 32000),   # two
+    (24, 5, 32000),   # two where the sampled rule has one
+    (24, 5, 29999),   # two, one value at a time
+    (16, 5, 50256),   # three
+    (16, 5, 50257),   # four
+    (12, 5, 75000),   # five of exactly 15,000
+    (12, 5, 74996),   # four
+    (30, 5, 60000),   # two: 330 rows
+])
+def test_greedy_rows_in_pieces(cuda, B, gamma, V):
+    """Each row's largest value twice, in different pieces or at their edges: the
+    first index counts."""
+    g = torch.Generator().manual_seed(B + V)
+    z = torch.randn(B, 2 * gamma + 1, V, generator=g)
+    edges = [V * k // n for n in (2, 3, 4, 5) for k in range(n)] + [V - 1]
+    for row in z.reshape(-1, V):
+        i = [edges[int(k)] - int(o) for k, o in zip(torch.randint(0, len(edges), (2,), generator=g),
+                                                    torch.randint(0, 2, (2,), generator=g))]
+        row[i] = 9.0  # (index -1: the last value)
+    target, draft = z[:, :gamma + 1].contiguous(), z[:, gamma + 1:].contiguous()
+    x = target[:, :gamma].argmax(-1).int()
+    x[:, -1] = draft[:, -1].argmax(-1).int()
+    u = torch.rand(B, gamma, generator=g)
+    want = S.verify_from_logits(target, draft, x, u, torch.ones(B, V), 0.0)
+    res = es.verify_sample(target.to(cuda), draft.to(cuda), x.to(cuda), u.to(cuda), None, 0.0)
+    assert res.accepted_lists() == want
