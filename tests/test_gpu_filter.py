@@ -31,6 +31,7 @@ import torch
 from engine import _hip
 from engine import spec_scheduler as es
 from oracle import sampler as S
+from oracle import spec_step as ref_step
 from specdec import sampler as gs
 from specdec.config import SamplingConfig
 
@@ -292,3 +293,45 @@ def test_both_zeros_tie_at_the_kth_value(cuda, T, top_k, above):
     got = es.verify_sample(z.to(cuda), draft.to(cuda), x.to(cuda), u.to(cuda), noise.to(cuda), T, top_k=top_k)
     assert got.accepted_lists() == S.verify_from_logits(z, draft, x, u, noise, T, top_k, 1.0)
     assert all(t[-1] == int(minus[3]) for t in got.accepted_lists())
+
+
+@pytest.mark.parametrize("mixed", [False, True])
+@pytest.mark.parametrize("top_p", [1.0, 0.9])
+@pytest.mark.parametrize("eos,budget", [(None, True), (3, True), (3, False), (None, False)])
+def test_commit_of_filtered_sampling_matches_oracle(cuda, eos, budget, top_p, mixed):
+    """Start positions, budgets (zero and negative ones too) and an eos among the
+    accepted tokens or drawn, in the one-launch form; ``mixed``: every third sequence
+    has 2,992 ties at the k-th value, which the general kernels commit."""
+    B, gamma, vocab, top_k = 36, 4, 3000, 8
+    g = torch.Generator().manual_seed(22 + int(10 * top_p))
+    target = torch.randn(B, gamma + 1, vocab, generator=g) - 8.0
+    target[..., :8] += 8.0  # eight likely tokens, the eos among them
+    draft = target[:, :gamma] + 0.3 * torch.randn(B, gamma, vocab, generator=g)
+    if mixed:
+        target[1::3, 0, 8:] = -12.0
+        target[1::3, 0, 5:8] = -13.0
+    q = S.logits_to_probs(draft, 1.0, top_k, top_p)
+    x = torch.multinomial(q.reshape(-1, vocab), 1, generator=g).reshape(B, gamma)
+    u = torch.rand(B, gamma, generator=g)
+    noise = torch.empty(B, vocab).exponential_(1, generator=g)
+    start = torch.randint(10, 100, (B,), generator=g)
+    remaining = torch.randint(1, 7, (B,), generator=g)
+    remaining[:8] = torch.tensor([0, 0, -1, -1, -2, -2, 1, 1])  # both kinds of sequence
+    want = S.verify_from_logits(target, draft, x, u, noise, 1.0, top_k, top_p)
+    res = es.verify_sample(target.to(cuda), draft.to(cuda), x.to(cuda), u.to(cuda), noise.to(cuda), 1.0,
+                           start_pos=start.to(cuda), remaining=remaining.to(cuda) if budget else None, eos_id=eos,
+                           top_k=top_k, top_p=top_p)
+    n_commit, fin, new_len = res.n_commit.tolist(), res.finished.tolist(), res.new_len.tolist()
+    flags, hits = res.flags.tolist(), [0, 0]
+    assert flags.count(0) >= B - 6
+    for b, got in enumerate(res.accepted_lists()):
+        assert got == want[b] or flags[b], b
+        rem = int(remaining[b]) if budget else len(got)
+        kept, eos_hit = ref_step.cut_accepted(got, rem, eos)
+        k = len(kept)
+        assert n_commit[b] == k, b
+        assert fin[b] == int(eos_hit or k == 0 or (budget and k >= rem)), b
+        assert new_len[b] == (int(start[b]) + k if k > 0 else -1), b
+        if eos_hit:
+            hits[k == len(got) - 1] += 1
+    assert eos is None or min(hits) > 0  # an eos among the accepted tokens, and drawn
