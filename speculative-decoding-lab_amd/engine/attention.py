@@ -129,20 +129,25 @@ def append_verify_attention(query_3d: torch.Tensor, k_new: torch.Tensor, v_new: 
     shape (``spv_verify_attn_append_planned``); the two calls otherwise."""
     B, chunk, hq, d = query_3d.shape
     shape = (B, chunk, kv.num_kv_heads, d)
-    # ``out`` must not overlap the new keys / values: some workgroups write it
-    # while others still read them.
     if (B and plan.buf is not None and write_plan.ready and not kv.fp8 and d == kv.head_dim
             and kv._plannable(chunk) and query_3d.device == kv.device
             and tuple(k_new.shape) == shape and tuple(v_new.shape) == shape
-            and k_new.device == kv.device and v_new.device == kv.device
-            and (out is None or not {k_new.untyped_storage().data_ptr(), v_new.untyped_storage().data_ptr()}
-                 & {out.untyped_storage().data_ptr()})):
-        write_plan._check(kv.allocator.epoch, B, chunk, seq_ids, start_positions)
+            and k_new.device == kv.device and v_new.device == kv.device):
         k_new, v_new = kv._new_kv(k_new, v_new)
-        return _attend(query_3d, kv, layer, seq_ids, start_positions, max_ctx, None, out, plan,
-                       (k_new, v_new, write_plan.rows))
+        # ``out`` must not overlap the new keys / values: some workgroups write it
+        # while others still read them.
+        if out is None or not (_overlap(out, k_new) or _overlap(out, v_new)):
+            write_plan._check(kv.allocator.epoch, B, chunk, seq_ids, start_positions)
+            return _attend(query_3d, kv, layer, seq_ids, start_positions, max_ctx, None, out, plan,
+                           (k_new, v_new, write_plan.rows))
     kv.write_block_device(layer, seq_ids, start_positions, k_new, v_new, alloc=False, plan=write_plan)
     return verify_attention(query_3d, kv, layer, seq_ids, start_positions, max_ctx, out=out, plan=plan)
+
+
+def _overlap(a: torch.Tensor, b: torch.Tensor) -> bool:
+    """Whether two contiguous tensors share memory, through whatever storages."""
+    return (a.data_ptr() < b.data_ptr() + b.numel() * b.element_size()
+            and b.data_ptr() < a.data_ptr() + a.numel() * a.element_size())
 
 
 def _attend(query_3d, kv, layer, seq_ids, start_positions, max_ctx, scale, out, plan, append) -> torch.Tensor:

@@ -115,3 +115,26 @@ def test_output_over_the_new_keys(cuda):
         outs.append(append_verify_attention(q, k1, v, kv, 1, sid, st, 70 + C, plan, wplan,
                                             out=k1 if kv is b else None))
     assert torch.equal(outs[0], outs[1]) and _same(a.k_pool, b.k_pool)
+
+
+@pytest.mark.parametrize("which", ["keys", "values"])
+def test_output_over_the_new_keys_through_another_storage(cuda, which):
+    # half of the output lies over half of the new keys (values), in a storage of its own
+    lens, C = [40, 70, 9], 4
+    (a, b), g = _pools(cuda, lens, C, 2, 64, torch.bfloat16, 2, seed=8)
+    sid, st = _hip.i32([0, 1, 2], cuda), _hip.i32(lens, cuda)
+    q, k, v = (torch.randn(3, C, 2, 64, generator=g).to(torch.bfloat16).to(cuda) for _ in range(3))
+    n = q.numel()
+    outs = []
+    for kv in (a, b):
+        wplan = WritePlan()
+        kv.write_block_device(0, sid, st, k, v, alloc=True, plan=wplan)
+        plan = VerifyPlan(kv, sid, st, C, 2, 70 + C)
+        buf = torch.zeros(2 * n, dtype=torch.bfloat16, device=cuda)
+        new = buf[:n].copy_((k if which == "keys" else v).reshape(-1)).view_as(k)
+        out = torch.from_dlpack(buf[n // 2:n // 2 + n]).view_as(k)
+        assert out.untyped_storage().data_ptr() != new.untyped_storage().data_ptr()
+        kn, vn = (new, v) if which == "keys" else (k, new)
+        outs.append(append_verify_attention(q, kn, vn, kv, 1, sid, st, 70 + C, plan, wplan,
+                                            out=out if kv is b else None))
+    assert torch.equal(outs[0], outs[1]) and _same(a.k_pool, b.k_pool) and _same(a.v_pool, b.v_pool)
