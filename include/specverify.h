@@ -292,10 +292,13 @@ size_t spv_verify_attn_workspace_bytes(int32_t B, int32_t C, int32_t num_q_heads
  * head h / (Hq/Hkv) (attention.py:32-38). q/out are (B, C, Hq, d) in q_dtype
  * (f32/bf16/f16); the pool holds kv_dtype. For SPV_FP8E4M3 pools kv_scales is
  * [layers][capacity][2] fp32 (K, V scale of each block). max_ctx must be >=
- * start_b + C for every b. bf16 queries over bf16 or fp8 pools, and fp16
- * queries over fp16 pools, with head_dim 128 or 64, block_size 16 and
- * B <= 2048 take the MFMA path (any (Hq/Hkv)*C); everything else (including
- * larger batches and mixed bf16 / fp16 operands) the VALU path.
+ * start_b + C for every b. bf16 queries over bf16 or fp8 pools, fp16 queries
+ * over fp16 pools, and f32 queries over f32 pools, with head_dim 128 or 64,
+ * block_size 16 and B <= 2048 take the MFMA path (any (Hq/Hkv)*C); everything
+ * else (including larger batches and mixed operands) the VALU path. f32 calls
+ * need what the VALU path needs (nothing for the shortest contexts) and take it
+ * where the workspace is smaller than the MFMA path's partials; with more, they
+ * use the workspace's arrival counters and partials as the 16-bit types do.
  * seq_lens / ctr (the pool's, both may be NULL): a read the contract forbids
  * -- a table entry outside [0, capacity), start_b + C > seq_lens[seq_ids[b]]
  * (keys not written yet), start_b < 0 or start_b + C > max_ctx -- sets
@@ -352,7 +355,8 @@ int spv_verify_attn_planned(void* out, const void* q, int q_dtype,
  * over it (the write-then-attend order of engine/model.py:182-190), in one
  * launch where the planned kernels run over bf16 or fp16 pages: k_new / v_new
  * (B, C, Hkv, d) in kv_dtype go to the rows of write_plan first. Arguments and
- * limits are those of the two calls; k_new / v_new must not overlap out. */
+ * limits are those of the two calls; k_new / v_new must not overlap out (some
+ * workgroups write it while others still read them). */
 int spv_verify_attn_append_planned(void* out, const void* q, int q_dtype,
                                    void* k_pool, void* v_pool, int kv_dtype,
                                    const int32_t* block_tables, int32_t max_blocks_per_seq,
@@ -370,7 +374,8 @@ int spv_verify_attn_append_planned(void* out, const void* q, int q_dtype,
  * hipMalloc). The kernels keep their counters and partials in the library's
  * own static device array of spv_verify_attn_static_max_bytes() bytes (24 MiB;
  * one per GPU, held until the process ends); a call that needs more (see
- * spv_verify_attn_workspace_bytes: the VALU path with long split contexts) is
+ * spv_verify_attn_workspace_bytes: the VALU path with long split contexts, and
+ * f32 calls whose VALU path would) is
  * rejected with SPV_ERR_WORKSPACE before anything is enqueued. Every call on
  * one GPU shares that array: calls that overlap on a GPU (other streams,
  * other host threads) race and give wrong results; order them. Arguments and
@@ -472,7 +477,8 @@ int spv_verify_sample(const float* target, const float* draft, int is_probs,
  * first: logits_to_probs(z, T, top_k, top_p) of the target and draft logits,
  * T > 0, then the decisions, draw and commit of spv_verify_sample. The filters
  * are those of spv_filter_logits (top_k <= 0 or >= V, or top_p outside (0, 1):
- * that filter is off). With 0 < top_k <= 512 one launch keeps each row's
+ * that filter is off; +0.0 and -0.0 are equal). With 0 < top_k <= 512, T from
+ * 2^-10 to 2^10, at most 65,536 rows and V <= 655,296, one launch keeps each row's
  * survivors and makes the whole result; sequences it does not cover (a NaN or
  * infinite logit, more than 1,024 values kept by top-k, a noise entry that is
  * not above zero), and every other call, take spv_filter_logits' kernel into

@@ -232,7 +232,6 @@ __device__ __forceinline__ bool decision_in_band(double pd, double qd, double u,
 // float(max(T, 1e-12)) as the fp32 scalar torch divides by.
 inline float temperature_divisor(float T) { return (float)((double)T > kEps ? (double)T : kEps); }
 
-
 // ------------------------------------------------------- top-k / top-p filters
 // Half width of the window around the nucleus edge p W (relative to W) where
 // the reference's fp32 softmax and cumulative sum can keep or drop a value

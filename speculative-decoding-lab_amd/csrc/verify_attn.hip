@@ -275,7 +275,7 @@ __host__ __device__ constexpr int ring_depth(int, int, int) { return 2; }
 // head_dim 128; measured best among 24..56 at batch 128, 16/2 heads, contexts
 // log-uniform in [512, 8192], 2-3% ahead of 48, the best before the combine
 // and spill fixes), scaled to the page size.
-__host__ __device__ constexpr int piece_cost(int d, int kt) { 
+__host__ __device__ constexpr int piece_cost(int d, int kt) {
   return 32 * 8192 / (16 * d * 2 * (kt == SPV_FP8E4M3 ? 1 : kt == SPV_F32 ? 4 : 2));
 }
 constexpr int kMfmaThreads = 512;
@@ -2095,8 +2095,6 @@ int spv::verify_attn_impl(void* out, const void* q, int q_dtype, const void* k_p
   }
   return SPV_OK;
 }
-
-
 
 extern "C" {
 
