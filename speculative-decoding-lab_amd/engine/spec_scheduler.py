@@ -177,10 +177,11 @@ def verify_sample(target: torch.Tensor, draft: torch.Tensor, proposals: torch.Te
     probabilities with ``is_probs``); ``proposals`` (B, gamma); ``u`` (B, gamma)
     uniforms; ``noise`` (B, V) ``Exp(1)`` rows (unused for greedy logits).
     ``top_k``/``top_p`` filter both sides' logits first (logits_to_probs,
-    specdec/sampler.py:19-56; sampling mode only): every row is scaled and
-    filtered in one launch, then sampled at temperature 1; with top_p a
-    sequence whose rows have values within rounding of the nucleus edge gets
-    ``FLAG_TOP_P_BAND``. ``draft_stats`` (B, gamma, 2) float32: the draft
+    specdec/sampler.py:19-56; sampling mode only): with 0 < top_k <= 512 one
+    launch makes the result from each row's survivors, otherwise every row is
+    scaled and filtered, then sampled at temperature 1
+    (``spv_verify_sample_filtered``); with top_p a sequence whose rows have
+    values within rounding of the nucleus edge gets ``FLAG_TOP_P_BAND``. ``draft_stats`` (B, gamma, 2) float32: the draft
     rows' statistics as ``draft_sample`` / ``DraftLoop`` wrote them when they
     drew the proposals at this temperature (the draft loop's q,
     spec_scheduler.py:243-252), so only the target rows are read for their
