@@ -121,7 +121,7 @@ __global__ __launch_bounds__(kFThreads) void filter_rows_kernel(FilterArgs a) {
     mx = s_red[0];
     for (int w = 1; w < kFThreads / 64; ++w) mx = fmaxf(mx, s_red[w]);
   };
-  float ml = 0.f;
+  float mz = 0.f;  // the maximum, 0 in a row with nothing finite
 
   // Histogram of one radix level: digit d of the keys >= min_key that match
   // (prefix, pmask) at `shift` with `nbits` bits, in `ncopy` copies; counts,
@@ -142,7 +142,7 @@ __global__ __launch_bounds__(kFThreads) void filter_rows_kernel(FilterArgs a) {
       if (key < min_key || (key & pmask) != prefix) return;
       const int d = (int)((key >> shift) & dmask);
       atomicAdd(&s_cnt[copy + d], 1);
-      if (by_mass) atomicAdd(&s_mass[copy + d], (double)__builtin_amdgcn_exp2f(fmaf(x, kLog2e, -ml)));
+      if (by_mass) atomicAdd(&s_mass[copy + d], mass_of(x, mz));
     });
     __syncthreads();
   };
@@ -287,7 +287,7 @@ __global__ __launch_bounds__(kFThreads) void filter_rows_kernel(FilterArgs a) {
   }
   if (do_p) {
     reduce_max();
-    ml = mx == -INFINITY ? 0.f : mx * kLog2e;
+    mz = mx == -INFINITY ? 0.f : mx;
     // Among what top-k kept (keys >= thr), by mass: search 0 finds the value
     // that crosses p W (W: the kept mass); with a window count asked for,
     // searches 1 and 2 find the values that cross (p -+ kTopPWindow) W. The
@@ -326,7 +326,7 @@ __global__ __launch_bounds__(kFThreads) void filter_rows_kernel(FilterArgs a) {
     const uint32_t tkey = pre[0];
     const double above = abv[0];
     const int total_ties = s_mdcnt[0];  // the last level's selected bin: the keys equal to tkey
-    const double wt = key_mass(tkey, ml);
+    const double wt = key_mass(tkey, mz);
     long long c = total_ties;
     if (wt > 0.0) {
       const double need_c = ceil((s_tgt[0] - above) / wt);
@@ -335,7 +335,7 @@ __global__ __launch_bounds__(kFThreads) void filter_rows_kernel(FilterArgs a) {
     if (ambiguous && tid == 0) {
       // Sorted position of the value crossing target t: c_t - 1 ties into its key.
       auto cross_pos = [&](int t) -> long long {
-        const double w = key_mass(pre[t], ml);
+        const double w = key_mass(pre[t], mz);
         long long j = s_mdcnt[t] - 1;
         if (w > 0.0) {
           const double need_t = ceil((s_tgt[t] - abv[t]) / w) - 1.0;

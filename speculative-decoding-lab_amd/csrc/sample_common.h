@@ -251,10 +251,12 @@ __device__ __forceinline__ float key_value(uint32_t k) {
   return __uint_as_float((k & 0x80000000u) ? (k & 0x7fffffffu) : ~k);
 }
 
-// The fp64 mass exp(x - max) of a key's value, as the histograms sum it.
-__device__ __forceinline__ double key_mass(uint32_t k, float ml) {
-  return (double)__builtin_amdgcn_exp2f(fmaf(key_value(k), kLog2e, -ml));
+// The mass exp(x - max) of a value, as fp64 sums take it. (x - max first: max
+// log2 e overflows in a row whose largest value is a mask's, the type's lowest.)
+__device__ __forceinline__ double mass_of(float x, float mx) {
+  return (double)__builtin_amdgcn_exp2f((x - mx) * kLog2e);
 }
+__device__ __forceinline__ double key_mass(uint32_t k, float mx) { return mass_of(key_value(k), mx); }
 
 // Block-wide exclusive scan of one double per thread (bins in descending order).
 __device__ __forceinline__ double block_exclusive_scan_f64(double v, double* lds, double* total) {

@@ -542,16 +542,15 @@ __global__ __launch_bounds__(kTThreads, NVEC == kVecMid ? 4 : 2) void topk_sampl
         const int per = (nk + kTThreads - 1) / kTThreads, q0 = min(nk, t * per), q1 = min(nk, q0 + per);
         if (a.top_p > 0.f && a.top_p < 1.f) {
           // the nucleus: a value stays while the mass before it is below p W
-          const float ml = M * kLog2e;
           double mine = 0.0, W;
-          for (int q = q0; q < q1; ++q) mine += key_mass(entry_key(s_row[q]), ml);
+          for (int q = q0; q < q1; ++q) mine += key_mass(entry_key(s_row[q]), M);
           double before = block_exclusive_scan_f64(mine, s_scan, &W);
           const double tgt = (double)a.top_p * W, lo = tgt - kTopPWindow * W, hi = tgt + kTopPWindow * W;
           int kept = 0, near = 0;
           for (int q = q0; q < q1; ++q) {
             kept += before < tgt;
             near += before >= lo && before < hi;
-            before += key_mass(entry_key(s_row[q]), ml);
+            before += key_mass(entry_key(s_row[q]), M);
           }
           // the masses before them rise with the rank: the kept values come first
           keep = max(1, block_sum(kept, s_cnt));

@@ -335,3 +335,26 @@ def test_commit_of_filtered_sampling_matches_oracle(cuda, eos, budget, top_p, mi
         if eos_hit:
             hits[k == len(got) - 1] += 1
     assert eos is None or min(hits) > 0  # an eos among the accepted tokens, and drawn
+
+
+@pytest.mark.parametrize("top_k", [0, 5])
+@pytest.mark.parametrize("top", [-2.5e38, -3.4e38, torch.finfo(torch.float32).min])
+def test_rows_masked_with_the_lowest_value(cuda, top, top_k):
+    """A row whose largest value times log2 e is beyond fp32: three values share the
+    mass, the others (the type's lowest, or nothing at all) have none."""
+    vocab, low = 900, torch.finfo(torch.float32).min
+    z = torch.full((2, 2, vocab), low if top > low else float("-inf"))
+    z[..., [7, 300, 899]] = top
+    want = S.filter_logits(z, 1.0, top_k, 0.9)
+    assert int(torch.isfinite(want).sum()) == 3 * 4
+    got, near = _hip.filter_rows(z.to(cuda), 1.0, top_k, 0.9, ambiguous=True)
+    assert torch.equal(got.cpu(), want) and not bool(near.any())
+    if top_k:  # the one-launch form
+        x = torch.tensor([[7], [300]], dtype=torch.int32)
+        u, noise = torch.tensor([[0.5], [0.5]]), torch.ones(2, vocab)
+        noise[0, 899] = noise[1, 7] = 0.25
+        draft = z[:, :1].contiguous()
+        res = es.verify_sample(z.to(cuda), draft.to(cuda), x.to(cuda), u.to(cuda), noise.to(cuda), 1.0,
+                               top_k=top_k, top_p=0.9)
+        assert res.accepted_lists() == S.verify_from_logits(z, draft, x, u, noise, 1.0, top_k, 0.9) == [[7, 899], [300, 7]]
+        assert res.flags.tolist() == [0, 0]
