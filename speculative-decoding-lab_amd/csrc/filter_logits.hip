@@ -281,7 +281,8 @@ __global__ __launch_bounds__(kFThreads) void filter_rows_kernel(FilterArgs a) {
       count_level(kShift[lv], kLBits[lv], kLCopies[lv], do_p && lv == 0, need);
       need = s_need;
     }
-    thr = prefix;  // the k-th largest key: every key >= it stays
+    // the k-th largest key: every key >= it stays (a NaN: nothing is below it)
+    thr = prefix == 0xffffffffu ? 0u : prefix;
   } else if (do_p) {
     for_row<UNIT>(z, V, tf, [&](int, float x) { mx = fmaxf(mx, x); });
   }
@@ -320,6 +321,9 @@ __global__ __launch_bounds__(kFThreads) void filter_rows_kernel(FilterArgs a) {
       // first pass resets them
       __syncthreads();
     }
+    // A NaN or +inf among the kept values leaves W without a value: as in the
+    // reference's softmax and cumulative sum, nothing is masked then.
+    const bool no_mass = isnan(s_tgt[0]);
     // pre[0]: the key of the value that crosses p; abv[0]: mass of larger
     // values. Its ties (equal value, equal mass) stay while the mass before
     // them is below the target: c of them, in ascending index order.
@@ -328,7 +332,7 @@ __global__ __launch_bounds__(kFThreads) void filter_rows_kernel(FilterArgs a) {
     const int total_ties = s_mdcnt[0];  // the last level's selected bin: the keys equal to tkey
     const double wt = key_mass(tkey, mz);
     long long c = total_ties;
-    if (wt > 0.0) {
+    if (wt > 0.0 && !no_mass) {
       const double need_c = ceil((s_tgt[0] - above) / wt);
       c = need_c < 1.0 ? 1 : (need_c > (double)total_ties ? total_ties : (long long)need_c);
     }
@@ -337,7 +341,7 @@ __global__ __launch_bounds__(kFThreads) void filter_rows_kernel(FilterArgs a) {
       auto cross_pos = [&](int t) -> long long {
         const double w = key_mass(pre[t], mz);
         long long j = s_mdcnt[t] - 1;
-        if (w > 0.0) {
+        if (w > 0.0 && !no_mass) {
           const double need_t = ceil((s_tgt[t] - abv[t]) / w) - 1.0;
           j = need_t < 0.0 ? 0 : (need_t > (double)(s_mdcnt[t] - 1) ? s_mdcnt[t] - 1 : (long long)need_t);
         }
@@ -347,9 +351,9 @@ __global__ __launch_bounds__(kFThreads) void filter_rows_kernel(FilterArgs a) {
       // after the value crossing the lower edge to the one crossing the upper.
       const long long lo = s_tgt[1] <= 0.0 ? 0 : cross_pos(1) + 1;
       const long long hi = cross_pos(2);
-      ambiguous[row] = hi >= lo ? (int)(hi - lo + 1) : 0;
+      ambiguous[row] = hi >= lo && !no_mass ? (int)(hi - lo + 1) : 0;
     }
-    thr = tkey;
+    thr = no_mass ? min_key : tkey;
     if (c < total_ties) {
       // the c-th tie in index order: each thread counts the ties of its own
       // contiguous span of the row, then the span holding it walks its elements

@@ -358,3 +358,28 @@ def test_rows_masked_with_the_lowest_value(cuda, top, top_k):
                                top_k=top_k, top_p=0.9)
         assert res.accepted_lists() == S.verify_from_logits(z, draft, x, u, noise, 1.0, top_k, 0.9) == [[7, 899], [300, 7]]
         assert res.flags.tolist() == [0, 0]
+
+
+@pytest.mark.parametrize("top_k,top_p", [(0, 0.9), (0, 1e-6), (3, 0.5), (1, 1.0), (2, 0.99)])
+@pytest.mark.parametrize("odd", ["nan", "two nans", "inf", "inf and nan", "-inf row"])
+def test_rows_without_a_mass(cuda, odd, top_k, top_p):
+    """The masses of a row with a NaN or +inf have no value: nothing is masked by
+    them, as in the reference; a NaN at the k-th place drops nothing."""
+    for vocab in (5, 300, 5000):
+        z = torch.randn(4, vocab, generator=torch.Generator().manual_seed(vocab)).round()  # ties
+        if "nan" in odd:
+            z[1, 3] = float("nan")
+        if odd == "two nans":
+            z[1, vocab - 1] = float("nan")
+        if "inf" in odd:
+            z[2, 1] = float("inf")
+        if odd == "-inf row":
+            z[2] = float("-inf")
+        want = S.filter_logits(z, 1.0, top_k, top_p)
+        for _ in range(3):
+            got, near = _hip.filter_rows(z.to(cuda), 1.0, top_k, top_p, ambiguous=True)
+            for b, whole in ((1, "nan" in odd), (2, "inf" in odd)):
+                if whole:
+                    assert torch.equal(got[b].cpu().nan_to_num(7.5), want[b].nan_to_num(7.5)), (vocab, b)
+                    assert int(near[b]) == 0 or odd == "-inf row"
+            assert torch.equal(got[0].isfinite().sum().cpu(), want[0].isfinite().sum())
