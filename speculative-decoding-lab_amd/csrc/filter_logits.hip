@@ -282,7 +282,7 @@ __global__ __launch_bounds__(kFThreads) void filter_rows_kernel(FilterArgs a) {
       need = s_need;
     }
     // the k-th largest key: every key >= it stays (a NaN: nothing is below it)
-    thr = prefix == 0xffffffffu ? 0u : prefix;
+    thr = prefix == 0xffffffffu ? 0u : with_both_zeros(prefix);
   } else if (do_p) {
     for_row<UNIT>(z, V, tf, [&](int, float x) { mx = fmaxf(mx, x); });
   }

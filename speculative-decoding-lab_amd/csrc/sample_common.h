@@ -239,13 +239,17 @@ inline float temperature_divisor(float T) { return (float)((double)T > kEps ? (d
 // row is off by up to ~1e-5, and the cumulative sum rounds each entry.
 constexpr double kTopPWindow = 5e-5;
 
-// Larger x, larger key; NaN above everything (torch.topk ranks NaN first). Both
-// zeros have the key of +0.0: they are equal to the filters' float comparisons.
+// Larger x, larger key; NaN above everything (torch.topk ranks NaN first).
 __device__ __forceinline__ uint32_t order_key(float x) {
-  const uint32_t u = __float_as_uint(x + 0.f);
+  const uint32_t u = __float_as_uint(x);
   if (x != x) return 0xffffffffu;
   return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }
+
+// A top-k bound: +0.0 ranks above -0.0, which the filter's float comparison does
+// not drop either. (One key for both zeros in order_key itself cost 2-3 us a call
+// at top_k 512, and 1% of the general filter.)
+__device__ __forceinline__ uint32_t with_both_zeros(uint32_t key) { return key == 0x80000000u ? 0x7fffffffu : key; }
 
 __device__ __forceinline__ float key_value(uint32_t k) {
   return __uint_as_float((k & 0x80000000u) ? (k & 0x7fffffffu) : ~k);

@@ -510,6 +510,7 @@ __global__ __launch_bounds__(kTThreads, NVEC == kVecMid ? 4 : 2) void topk_sampl
       };
       find(false);
       if (held > kKeepCap) find(true);
+      thr = with_both_zeros(thr);
       if (t == 0) s_n = 0;
       __syncthreads();
       for (int i = t; i < total; i += kTThreads) {
@@ -532,9 +533,9 @@ __global__ __launch_bounds__(kTThreads, NVEC == kVecMid ? 4 : 2) void topk_sampl
         }
         __syncthreads();
         if (thr && nk > a.top_k) {  // cut at the k-th value; its ties stay
-          const uint32_t kth = entry_key(s_row[a.top_k - 1]);
+          const uint32_t kth = with_both_zeros(entry_key(s_row[a.top_k - 1]));
           int ties = 0;
-          for (int i = a.top_k + t; i < nk; i += kTThreads) ties += entry_key(s_row[i]) == kth;
+          for (int i = a.top_k + t; i < nk; i += kTThreads) ties += entry_key(s_row[i]) >= kth;
           nk = a.top_k + block_sum(ties, s_cnt);
         }
         const float M = key_value(entry_key(s_row[0]));
